@@ -1,7 +1,6 @@
 // extern "C" entry points of libace_hip.so (declared in include/ace_hip.h).
 //
-// Host side of the boundary: argument validation, launch geometry, the
-// alignment test that selects vector loads, and dispatch to the kernel
+// Host side of the boundary: argument validation, launch geometry and dispatch to the kernel
 // instantiation for (element type, binning, channel variant).  No call
 // allocates, copies or synchronises.
 #include <hip/hip_runtime.h>
@@ -228,10 +227,9 @@ FwdParams fwd_params(const void* x, int x_dtype, const void* target, bool labels
                      const float* class_weight, const float* bin_table, const float* centre_table,
                      void* workspace, const Geometry& g, float* coef, float* diff, float* jac,
                      float* per_class, float* loss, double* stats) {
-  const int vec = g.var.vec;
   const size_t es = elem_size(x_dtype);
-  const bool vec_ok = (voxels % vec) == 0 && aligned_to(x, es * vec) &&
-                      (labels ? aligned_to(target, 16) : aligned_to(target, 4 * vec));
+  // vector loads take any element (load_vec)
+  const bool vec_ok = aligned_to(x, es) && aligned_to(target, labels ? 8 : 4);
 
   FwdParams p{};
   p.x = x;
@@ -294,11 +292,9 @@ BwdParams bwd_params(const void* x, int x_dtype, const void* target, bool labels
                      const float* bin_table, const float* centre_table, const float* coef,
                      const float* diff, const float* jac, const float* grad_output,
                      int grad_output_per_class, void* dx, const Geometry& g) {
-  const int vec = g.var.vec;
   const size_t es = elem_size(x_dtype);
-  bool vec_ok = (voxels % vec) == 0 && aligned_to(x, es * vec) && aligned_to(dx, es * vec);
-  if (soft && target)
-    vec_ok = vec_ok && (labels ? aligned_to(target, 16) : aligned_to(target, 4 * vec));
+  bool vec_ok = aligned_to(x, es) && aligned_to(dx, es);
+  if (soft && target) vec_ok = vec_ok && aligned_to(target, labels ? 8 : 4);
 
   BwdParams p{};
   p.x = x;

@@ -158,50 +158,61 @@ template <> __device__ __forceinline__ __half from_f32<__half>(float v) {
   return __float2half(v);  // round to nearest even
 }
 
-template <int BYTES> struct RawVec;
-template <> struct RawVec<16> { using type = uint4; };
-template <> struct RawVec<8> { using type = uint2; };
-template <> struct RawVec<4> { using type = unsigned int; };
-template <> struct RawVec<2> { using type = unsigned short; };
+// VEC elements of T as one clang vector of 32-bit (or one narrower) words,
+// aligned like a single element: gfx950 takes a global load or store of any
+// width at any address (unaligned access mode, which HSA always sets), so
+// rows of any length and any starting element are read and written with full
+// vectors -- one global_load_dwordx4 where 16-byte alignment used to be the
+// condition and single elements the alternative.  A row off by an element
+// costs one more 128-byte line per 1 KiB wave request: the hard forward of
+// 1 x 4 x 191 x 223 x 207 float32 (211 MB, odd rows) went from 70.0 to
+// 55.8 us.
+template <int BYTES, int ALIGN> struct RawVec;
+#define ACE_RAW_VEC(BYTES, ALIGN, WORD, ...)                         \
+  template <> struct RawVec<BYTES, ALIGN> {                          \
+    typedef WORD type __attribute__((__VA_ARGS__, aligned(ALIGN)));  \
+  };
+ACE_RAW_VEC(16, 4, unsigned int, ext_vector_type(4))
+ACE_RAW_VEC(8, 4, unsigned int, ext_vector_type(2))
+ACE_RAW_VEC(8, 2, unsigned int, ext_vector_type(2))
+ACE_RAW_VEC(4, 4, unsigned int, may_alias)
+ACE_RAW_VEC(4, 2, unsigned int, may_alias)
+ACE_RAW_VEC(2, 2, unsigned short, may_alias)
+#undef ACE_RAW_VEC
+// Two int64 labels at the alignment of one.
+typedef long long xi64x2 __attribute__((ext_vector_type(2), aligned(8)));
 
-// The same widths as clang vector types, which the nontemporal store builtin
-// takes (global_store with the nt bit).
-typedef unsigned int xu32x4 __attribute__((ext_vector_type(4)));
-typedef unsigned int xu32x2 __attribute__((ext_vector_type(2)));
-template <int BYTES> struct XVec { using type = typename RawVec<BYTES>::type; };
-template <> struct XVec<16> { using type = xu32x4; };
-template <> struct XVec<8> { using type = xu32x2; };
-// VEC consecutive elements from an address aligned to VEC * sizeof(T).
+// VEC consecutive elements, at any element.
 template <typename T, int VEC>
 __device__ __forceinline__ void load_vec(const T* __restrict__ p, float (&out)[VEC]) {
-  using R = typename RawVec<sizeof(T) * VEC>::type;
+  using R = typename RawVec<sizeof(T) * VEC, sizeof(T)>::type;
   const R raw = *reinterpret_cast<const R*>(p);
   T vals[VEC];
-  __builtin_memcpy(vals, &raw, sizeof(R));
+  __builtin_memcpy(vals, &raw, sizeof(T) * VEC);
 #pragma unroll
   for (int j = 0; j < VEC; ++j) out[j] = to_f32<T>(vals[j]);
 }
 
 template <typename T, int VEC>
 __device__ __forceinline__ void store_vec(T* __restrict__ p, const float (&in)[VEC]) {
-  using R = typename RawVec<sizeof(T) * VEC>::type;
+  using R = typename RawVec<sizeof(T) * VEC, sizeof(T)>::type;
   T vals[VEC];
 #pragma unroll
   for (int j = 0; j < VEC; ++j) vals[j] = from_f32<T>(in[j]);
   R raw;
-  __builtin_memcpy(&raw, vals, sizeof(R));
+  __builtin_memcpy(&raw, vals, sizeof(T) * VEC);
   *reinterpret_cast<R*>(p) = raw;
 }
 
 // store_vec with a nontemporal store (streamed past the caches).
 template <typename T, int VEC>
 __device__ __forceinline__ void store_vec_nt(T* __restrict__ p, const float (&in)[VEC]) {
-  using R = typename XVec<sizeof(T) * VEC>::type;
+  using R = typename RawVec<sizeof(T) * VEC, sizeof(T)>::type;
   T vals[VEC];
 #pragma unroll
   for (int j = 0; j < VEC; ++j) vals[j] = from_f32<T>(in[j]);
   R raw;
-  __builtin_memcpy(&raw, vals, sizeof(R));
+  __builtin_memcpy(&raw, vals, sizeof(T) * VEC);
   __builtin_nontemporal_store(raw, reinterpret_cast<R*>(p));
 }
 // A gradient store: nontemporal for streaming problems (stream_problem).
@@ -218,14 +229,14 @@ __device__ __forceinline__ int label_channel(long long v, int C) {
   return (v >= 0 && v < (long long)C) ? (int)v : -1;
 }
 
-// VEC labels from an address aligned to 16 bytes (VEC even) or one label.
+// VEC labels (VEC even: two per 16-byte load) or one.
 template <int VEC>
 __device__ __forceinline__ void load_labels(const long long* __restrict__ p, int C,
                                             int (&lab)[VEC]) {
   if constexpr (VEC % 2 == 0) {
 #pragma unroll
     for (int j = 0; j < VEC; j += 2) {
-      const longlong2 t = *reinterpret_cast<const longlong2*>(p + j);
+      const xi64x2 t = *reinterpret_cast<const xi64x2*>(p + j);
       lab[j] = label_channel(t.x, C);
       lab[j + 1] = label_channel(t.y, C);
     }
@@ -235,8 +246,7 @@ __device__ __forceinline__ void load_labels(const long long* __restrict__ p, int
   }
 }
 
-// VEC consecutive elements, vector load when VEC > 1 (caller guarantees
-// alignment) or one element.
+// VEC consecutive elements (a vector load when VEC > 1) or one element.
 template <typename T, int VEC>
 __device__ __forceinline__ void load_row(const T* __restrict__ p, float (&out)[VEC]) {
   if constexpr (VEC > 1) {
@@ -1615,12 +1625,11 @@ __device__ __forceinline__ void fast_load(FastTile<C, VEC>& t, const T* const (&
 #pragma unroll
       for (int j = 0; j < VEC; j += 2) {
         if constexpr (NTL) {
-          typedef long long xi64x2 __attribute__((ext_vector_type(2)));
           const xi64x2 q = __builtin_nontemporal_load(reinterpret_cast<const xi64x2*>(lr + v + j));
           t.lab[j] = q.x;
           t.lab[j + 1] = q.y;
         } else {
-          const longlong2 q = *reinterpret_cast<const longlong2*>(lr + v + j);
+          const xi64x2 q = *reinterpret_cast<const xi64x2*>(lr + v + j);
           t.lab[j] = q.x;
           t.lab[j + 1] = q.y;
         }
@@ -2380,8 +2389,7 @@ hipError_t launch(Kern kern, long long nblk, size_t lds, hipStream_t s, const Pa
 template <typename T, int CMAX, bool EXACT, int VEC, bool SOFT, bool RIGHT>
 hipError_t launch_fwd_t(const Geometry& g, const FwdParams& prm, hipStream_t s) {
   // the geometry's voxels per lane (tiles, the alignment test behind
-  // vec_ok) must be the kernel's: a wider kernel would issue vector loads
-  // the host never checked
+  // vec_ok) must be the kernel's
   if (g.var.vec != VEC) return hipErrorInvalidConfiguration;
   auto kern = fwd_kernel<T, CMAX, EXACT, VEC, SOFT, RIGHT>;
   int nt = kThreads;
