@@ -13,6 +13,7 @@
 #include <mutex>
 
 #include "ace_core.hpp"
+#include "ace_wide.hpp"
 #include "ace_hip.h"
 
 namespace ace {
@@ -35,15 +36,28 @@ ACE_DECLARE_BOTH(__half, true)
 #undef ACE_DECLARE_BOTH
 #undef ACE_DECLARE_LAUNCHERS
 
+#define ACE_DECLARE_WIDE(T, SOFT)                                                                  \
+  template <> hipError_t launch_wide_fwd<T, SOFT>(const Geometry&, const FwdParams&, hipStream_t); \
+  template <> hipError_t launch_wide_bwd<T, SOFT>(const Geometry&, const BwdParams&, hipStream_t);
+ACE_DECLARE_WIDE(float, false)
+ACE_DECLARE_WIDE(float, true)
+ACE_DECLARE_WIDE(__hip_bfloat16, false)
+ACE_DECLARE_WIDE(__hip_bfloat16, true)
+ACE_DECLARE_WIDE(__half, false)
+ACE_DECLARE_WIDE(__half, true)
+#undef ACE_DECLARE_WIDE
+
 // Dispatch on (element type, binning, right) to the instantiated launchers.
 template <typename T>
 hipError_t pick_fwd(bool soft, bool right, const Geometry& g, const FwdParams& p, hipStream_t s) {
+  if (g.wide) return soft ? launch_wide_fwd<T, true>(g, p, s) : launch_wide_fwd<T, false>(g, p, s);
   if (soft)
     return right ? launch_variant_fwd<T, true, true>(g, p, s) : launch_variant_fwd<T, true, false>(g, p, s);
   return right ? launch_variant_fwd<T, false, true>(g, p, s) : launch_variant_fwd<T, false, false>(g, p, s);
 }
 template <typename T>
 hipError_t pick_bwd(bool soft, bool right, const Geometry& g, const BwdParams& p, hipStream_t s) {
+  if (g.wide) return soft ? launch_wide_bwd<T, true>(g, p, s) : launch_wide_bwd<T, false>(g, p, s);
   if (soft)
     return right ? launch_variant_bwd<T, true, true>(g, p, s) : launch_variant_bwd<T, true, false>(g, p, s);
   return right ? launch_variant_bwd<T, false, true>(g, p, s) : launch_variant_bwd<T, false, false>(g, p, s);
@@ -152,7 +166,7 @@ Geometry forward_geometry(int64_t batch, int64_t channels, int64_t voxels, int n
 }
 
 // The activation is not an argument here: the largest workspace of the
-// layouts a call may use (generic, fast, soft moments).
+// layouts a call may use (generic, fast, soft moments; wide_workspace_size).
 size_t workspace_size(int64_t batch, int64_t channels, int64_t voxels, int num_bins, int binning,
                       int include_background, int target_kind) {
   const bool soft = binning == ACE_SOFT;
@@ -168,6 +182,26 @@ size_t workspace_size(int64_t batch, int64_t channels, int64_t voxels, int num_b
     }
   }
   return best;
+}
+
+// The wide kernels' geometry of a problem, g.wide false where they do not serve
+// it: raw probabilities (no activation: values outside [0, 1]), too many soft
+// bins for the moments' fixed point, or an LDS layout that does not fit.  The
+// generic kernels keep those.
+Geometry wide_geometry(bool soft, bool labels, int act, int64_t batch, int64_t channels,
+                       int64_t voxels, int num_bins, int include_background) {
+  Geometry g{};
+  if (act == kActNone || channels > kMaxChannels || (soft && num_bins > kExactMaxBins)) return g;
+  g = make_wide_geometry(batch, channels, voxels, num_bins, soft, include_background != 0, labels);
+  g.wide = g.lds_fwd <= kMaxLds && g.lds_bwd <= kMaxLds && g.nblk <= 0x7fffffffLL;
+  return g;
+}
+
+size_t wide_workspace_size(int64_t batch, int64_t channels, int64_t voxels, int num_bins, int binning,
+                           int include_background, int target_kind) {
+  const Geometry g = wide_geometry(binning == ACE_SOFT, target_kind == ACE_TARGET_LABELS_I64, kActSigmoid,
+                                   batch, channels, voxels, num_bins, include_background);
+  return g.wide ? g.ws_bytes : 0;
 }
 
 // Vector steps per backward block: make_geometry's choice (~1024 blocks; 512 above 8 channels, where the forward's final-sum
@@ -187,7 +221,9 @@ int bwd_steps(bool soft, bool labels, int act, int64_t batch, int64_t channels, 
 
 // The forward's launch plan and the checks it must pass before anything is
 // launched: the geometry of the kernel the launcher will pick, within the
-// LDS and the grid's limits.
+// LDS and the grid's limits.  A wide kernel whose final sums do not fit in
+// ws_bytes of workspace (the moments hold ten words per bin, the generic soft
+// sums three) leaves the call to the generic kernel.
 struct ForwardPlan {
   int rc;
   int act;
@@ -195,12 +231,19 @@ struct ForwardPlan {
   Geometry g;
 };
 ForwardPlan plan_forward(int64_t batch, int64_t channels, int64_t voxels, int num_bins, int binning,
-                         int activation, int include_background, int target_kind) {
+                         int activation, int include_background, int target_kind, size_t ws_bytes) {
   ForwardPlan fp{};
   const bool soft = binning == ACE_SOFT;
   const bool labels = target_kind == ACE_TARGET_LABELS_I64;
   fp.act = (activation == ACE_ACT_SOFTMAX && channels == 1) ? kActNone : activation;
   fp.moments = use_moments(soft, labels, fp.act, batch, channels, voxels, num_bins, include_background);
+  if (!fast_forward(soft, labels, fp.act, channels, fp.moments)) {
+    fp.g = wide_geometry(soft, labels, fp.act, batch, channels, voxels, num_bins, include_background);
+    if (fp.g.wide && fp.g.ws_bytes <= ws_bytes) {
+      fp.moments = soft;
+      return fp;
+    }
+  }
   fp.g = forward_geometry(batch, channels, voxels, num_bins, soft, include_background, labels, fp.act,
                           fp.moments);
   fp.rc = (fp.g.lds_fwd > kMaxLds || fp.g.nblk > 0x7fffffffLL) ? ACE_EUNSUPPORTED : ACE_OK;
@@ -223,7 +266,8 @@ void set_fast_bins(FwdParams& p, int num_bins, int64_t channels) {
 // Kernel parameters of one forward problem (geometry g, workspace at ws).
 FwdParams fwd_params(const void* x, int x_dtype, const void* target, bool labels, int64_t voxels,
                      int64_t batch, int64_t channels, int num_bins, int act,
-                     int ignore_empty_classes, int reduction, float empty_weight, bool moments,
+                     int ignore_empty_classes, int reduction, int right, float empty_weight,
+                     bool moments,
                      const float* class_weight, const float* bin_table, const float* centre_table,
                      void* workspace, const Geometry& g, float* coef, float* diff, float* jac,
                      float* per_class, float* loss, double* stats) {
@@ -251,6 +295,7 @@ FwdParams fwd_params(const void* x, int x_dtype, const void* target, bool labels
   p.red = reduction;
   p.empty_w = empty_weight;
   p.packed = g.packed ? 1 : 0;
+  p.right = right;
   p.tl = g_timeline.load(std::memory_order_relaxed);
   p.max_polls = g_max_polls.load(std::memory_order_relaxed);
   p.publish_delay = g_publish_delay.load(std::memory_order_relaxed);
@@ -260,11 +305,12 @@ FwdParams fwd_params(const void* x, int x_dtype, const void* target, bool labels
   p.sscale = ldexp(1.0, -sf);
   if (g.fast && !moments) set_fast_bins(p, num_bins, channels);
   if (moments) {
-    const MomentScale ms = moment_scale(num_bins);
+    const MomentScale ms = g.wide ? exact_moment_scale(num_bins) : moment_scale(num_bins);
     p.msc = ldexpf(1.0f, ms.m);
     p.misc = ldexpf(1.0f, -ms.m);
     p.mw = ms.w;
-    p.mshift = moment_shift(voxels);
+    p.mshift = g.wide ? exact_moment_shift(voxels) : moment_shift(voxels);
+    p.mshift0 = exact_moment_shift0(voxels);
   }
   p.btab = bin_table;
   p.rtab = centre_table;
@@ -288,7 +334,7 @@ FwdParams fwd_params(const void* x, int x_dtype, const void* target, bool labels
 
 // Kernel parameters of one backward problem (geometry g).
 BwdParams bwd_params(const void* x, int x_dtype, const void* target, bool labels, bool soft,
-                     int64_t voxels, int64_t batch, int64_t channels, int num_bins, int act,
+                     int64_t voxels, int64_t batch, int64_t channels, int num_bins, int act, int right,
                      const float* bin_table, const float* centre_table, const float* coef,
                      const float* diff, const float* jac, const float* grad_output,
                      int grad_output_per_class, void* dx, const Geometry& g) {
@@ -317,6 +363,7 @@ BwdParams bwd_params(const void* x, int x_dtype, const void* target, bool labels
   p.d = diff;
   p.jac = jac;
   p.go = grad_output;
+  p.right = right;
   p.stream = stream_problem(es * (size_t)batch * (size_t)channels * (size_t)voxels,
                             target_bytes(labels, batch, channels, voxels)) ? 1 : 0;
 
@@ -476,8 +523,11 @@ size_t ace_workspace_bytes(int64_t batch, int64_t channels, int64_t voxels, int 
   if (batch < 1 || channels < 1 || voxels < 0 || num_bins < 1) return 0;
   if (x_dtype == ACE_F64)
     return f64::workspace_bytes(batch, channels, voxels, num_bins, binning, include_background);
-  return workspace_size(batch, channels, voxels, num_bins, binning, include_background,
-                        target_kind);
+  const size_t wide = wide_workspace_size(batch, channels, voxels, num_bins, binning,
+                                          include_background, target_kind);
+  const size_t rest = workspace_size(batch, channels, voxels, num_bins, binning, include_background,
+                                     target_kind);
+  return wide > rest ? wide : rest;
 }
 
 size_t ace_workspace_reset_bytes(int64_t batch, int64_t channels, int64_t voxels,
@@ -504,7 +554,7 @@ int ace_forward(const void* x, int x_dtype, const void* target, int target_kind,
   const bool soft = binning == ACE_SOFT;
   const bool labels = target_kind == ACE_TARGET_LABELS_I64;
   const ForwardPlan fp = plan_forward(batch, channels, voxels, num_bins, binning, activation,
-                                      include_background, target_kind);
+                                      include_background, target_kind, workspace_bytes);
   if (fp.rc) return fp.rc;
   const Geometry& g = fp.g;
   const int act = fp.act;
@@ -512,8 +562,8 @@ int ace_forward(const void* x, int x_dtype, const void* target, int target_kind,
   if (workspace_bytes < g.ws_bytes) return ACE_EWORKSPACE;
 
   const FwdParams p = fwd_params(x, x_dtype, target, labels, voxels, batch, channels, num_bins, act,
-                                  ignore_empty_classes, reduction, empty_weight, moments, class_weight,
-                                  bin_table, centre_table, workspace, g, coef, diff, jac, per_class,
+                                  ignore_empty_classes, reduction, right != 0, empty_weight, moments,
+                                  class_weight, bin_table, centre_table, workspace, g, coef, diff, jac, per_class,
                                   loss, stats);
   return to_code(dispatch_fwd(x_dtype, soft, right != 0, g, p, static_cast<hipStream_t>(stream)));
 }
@@ -534,16 +584,22 @@ int ace_backward(const void* x, int x_dtype, const void* target, int target_kind
   const int act = (activation == ACE_ACT_SOFTMAX && channels == 1) ? kActNone : activation;
   const bool moments =
       use_moments(soft, labels, act, batch, channels, voxels, num_bins, include_background);
-  const Geometry g = make_geometry(
-      batch, channels, voxels, num_bins, soft, include_background != 0, labels,
-      bwd_steps(soft, labels, act, batch, channels, voxels, include_background, moments), 0,
-      moments, false, kFastThreads, true);
+  // the fast kernels' calls as in the forward, and hard softmax gradients over
+  // their channel counts with any targets (they read none)
+  const bool fast = act == kActSoftmax && fast_channels(channels) && (!soft || moments);
+  Geometry g{};
+  if (!fast) g = wide_geometry(soft, labels, act, batch, channels, voxels, num_bins, include_background);
+  if (!g.wide)
+    g = make_geometry(
+        batch, channels, voxels, num_bins, soft, include_background != 0, labels,
+        bwd_steps(soft, labels, act, batch, channels, voxels, include_background, moments), 0,
+        moments, false, kFastThreads, true);
   if (g.lds_bwd > kMaxLds) return ACE_EUNSUPPORTED;
   if (g.nblk > 0x7fffffffLL) return ACE_EUNSUPPORTED;
   if (voxels == 0) return ACE_OK;
 
   const BwdParams p = bwd_params(x, x_dtype, target, labels, soft, voxels, batch, channels, num_bins,
-                                  act, bin_table, centre_table, coef, diff, jac, grad_output,
+                                  act, right != 0, bin_table, centre_table, coef, diff, jac, grad_output,
                                   grad_output_per_class, dx, g);
   return to_code(dispatch_bwd(x_dtype, soft, right != 0, g, p, static_cast<hipStream_t>(stream)));
 }
@@ -603,7 +659,7 @@ int ace_forward_levels(int levels, const AceFwdLevel* lv, int x_dtype, int64_t b
     if (g.nt != L.nt) return ACE_EUNSUPPORTED;
     if (nblk + g.nblk > 0x7fffffffLL) return ACE_EUNSUPPORTED;
     L.lv[l] = fwd_params(v.x, x_dtype, v.target, true, v.voxels, batch, channels, num_bins,
-                         kActSoftmax, ignore_empty_classes, reduction, empty_weight, moments,
+                         kActSoftmax, ignore_empty_classes, reduction, right != 0, empty_weight, moments,
                          class_weight, bin_table, centre_table,
                          static_cast<unsigned char*>(workspace) + off, g, v.coef, v.diff, v.jac,
                          v.per_class, v.loss, nullptr);
@@ -653,7 +709,7 @@ int ace_backward_levels(int levels, const AceBwdLevel* lv, int x_dtype, int64_t 
     if (g.lds_bwd > kMaxLds) return ACE_EUNSUPPORTED;
     if (nblk + g.nblk > 0x7fffffffLL) return ACE_EUNSUPPORTED;
     L.lv[l] = bwd_params(v.x, x_dtype, v.target, true, soft, v.voxels, batch, channels, num_bins,
-                         kActSoftmax, bin_table, centre_table, v.coef, v.diff, v.jac,
+                         kActSoftmax, right != 0, bin_table, centre_table, v.coef, v.diff, v.jac,
                          v.grad_output, grad_output_per_class, v.dx, g);
     L.start[l] = nblk;
     // a level with no voxels launches no blocks (ace_backward returns early)
@@ -689,13 +745,14 @@ int ace_forward_noalloc(const void* x, int x_dtype, const void* target, int targ
     return ACE_EINVAL;
   if (!coef || !diff || !jac || !per_class) return ACE_EINVAL;
   if (reduction != ACE_RED_NONE && !loss) return ACE_EINVAL;
-  rc = plan_forward(batch, channels, voxels, num_bins, binning, activation, include_background,
-                    target_kind).rc;
-  if (rc) return rc;
-  const size_t need = ace_workspace_reset_bytes(batch, channels, voxels, num_bins, binning, x_dtype,
-                                                include_background, target_kind);
-  if (need == 0) return ACE_EINVAL;
+  const ForwardPlan fp = plan_forward(batch, channels, voxels, num_bins, binning, activation,
+                                      include_background, target_kind, ACE_NOALLOC_SCRATCH_BYTES);
+  if (fp.rc) return fp.rc;
+  // every layout but the wide kernels', which give way where they do not fit
+  size_t need = workspace_size(batch, channels, voxels, num_bins, binning, include_background,
+                               target_kind);
   if (need > ACE_NOALLOC_SCRATCH_BYTES) return ACE_ESCRATCH;
+  if (fp.g.ws_bytes > need) need = fp.g.ws_bytes;
   void* ws = nullptr;
   rc = scratch_address(&ws);
   if (rc) return rc;

@@ -173,6 +173,47 @@ ACE_HD MomentScale moment_scale(int num_bins) {
   return s;
 }
 
+// Exact moments (the wide soft kernels, any p): the probabilities of half-bin
+// h are held as u = p 2^m - h w, exact in float32 and, for h >= 1, an integer
+// below 2^25:
+//   m = 23 + ceil(log2 2K): p > 1/2K (1 - 2^-14) there, whose spacing is at
+//   least 2^-m;
+//   ws = 2^m / 2K is in [2^23, 2^24), and w <= ws (1 - 2^-14) has at most
+//   24 - ceil(log2 2K) significant bits, so that h w is a float32 (h < 2K) and
+//   h w < e_h 2^m as in moment_scale.  w >= ws (1 - 2^-14 - 2^(c - 23)) with
+//   c = ceil(log2 2K), so u < ws (1 + 2K (2^-14 + 2^(c - 23) + 2^-21)) + 2K,
+//   below 1.2 2^24 for 2K <= 2^10 = 2 kExactMaxBins.
+//   u is a multiple of p 2^m's spacing (h w's is no finer where p 2^m >= 2^24),
+//   of at most 24 bits: fma(p, 2^m, -h w) is exact.
+// Half-bin 0 takes any p below 1/2K: both its weights fall into bin 0, so it
+// needs the sum of p alone, held to 2^-(m + 16).  The moments above quantise p
+// to 2^-m (m = 28 at 20 bins) by truncation instead, 2^-29 of p lost per voxel
+// on average.
+constexpr int kExactMaxBins = 512;
+ACE_HD MomentScale exact_moment_scale(int num_bins) {
+  int c = 0;
+  while ((1ll << c) < 2ll * num_bins) ++c;  // ceil(log2 2K)
+  MomentScale s;
+  s.m = 23 + c;
+  const double ws = (double)(1ll << s.m) / (2.0 * num_bins);
+  const int drop = c;  // ws (1 - 2^-14) takes 24 bits: keep 24 - c of them
+  s.w = ((int)(ws * (1.0 - 1.0 / 16384.0)) >> drop) << drop;
+  return s;
+}
+// Right shifts of its per-copy sums before the final sums of N voxels: u^2 <
+// 2^50.6 (a copy's 4095 voxels below 2^62.6), N 2^50.6 / 2^shift < 2^62.6; and
+// of half-bin 0's sums, 2^16 u < 2^40 a voxel.
+ACE_HD int exact_moment_shift(long long voxels) {
+  int bits = 0;
+  while (bits < 62 && (1ll << bits) <= voxels) ++bits;
+  return bits > 12 ? bits - 12 : 0;
+}
+ACE_HD int exact_moment_shift0(long long voxels) {
+  int bits = 0;
+  while (bits < 62 && (1ll << bits) <= voxels) ++bits;
+  return bits > 22 ? bits - 22 : 0;
+}
+
 // Right shift of the per-copy sums of u^2 before they are added into the
 // final sums of a batch index of N voxels: u^2 < 2^48, one copy holds at
 // most 4095 voxels (< 2^60), a block's tile fewer than 2^15 (below N unless

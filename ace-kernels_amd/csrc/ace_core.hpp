@@ -31,6 +31,8 @@
 #include <hip/hip_ext.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "ace_bins.hpp"
 #include "ace_geometry.hpp"
 
@@ -55,6 +57,11 @@ constexpr int kShiftG = 42;
 constexpr int kMomShiftN = 52;
 constexpr int kMomShiftG = 40;
 
+// How a forward kernel bins: per-bin sums; half-bin moments of quantised
+// probabilities (the fast soft kernels); exact half-bin moments (the wide
+// soft kernels, with class labels or with per-channel targets).
+enum { kMomNone = 0, kMomQuant = 1, kMomExact = 2, kMomExactTargets = 3 };
+
 struct FwdParams {
   const void* x;
   const void* tgt;
@@ -69,6 +76,7 @@ struct FwdParams {
   int epi_all;         // one block runs every batch index's epilogue and the loss
   float empty_w;
   int packed;          // hard binning with labels: final sums W << 32 | G, then P
+  int right;           // wide kernels: bucketize convention (others: a template argument)
   int max_polls;       // bound of the loss block's wait for a partial word (kMaxPolls)
   int publish_delay;   // test knob: sleeps before a batch epilogue publishes its word (0)
   // fast hard kernels (softmax + class labels, fast_bin): with n = K bins, a
@@ -87,6 +95,7 @@ struct FwdParams {
   float misc;          // 2^-m
   int mw;              // soft moments: half-bin h has base h mw (in units of 2^-m)
   int mshift;          // soft moments: right shift of the per-copy sums of u^2
+  int mshift0;         // the same for half-bin 0 of the exact moments
   const float* btab;   // bucket table (K or 2K upper boundaries)
   const float* rtab;   // soft centre table (2K + 2)
   const float* clsw;   // C' class weights or null
@@ -137,6 +146,7 @@ struct BwdParams {
   const float* d;
   const float* jac;
   const float* go;
+  int right;           // wide kernels, as in FwdParams
   int stream;          // streaming (nontemporal) gradient stores: stream_problem
 };
 
@@ -291,6 +301,18 @@ __device__ __forceinline__ unsigned long long square_u24(uint32_t u) {
   return ((unsigned long long)hi << 32) | lo;
 }
 
+// The second word of the exact moments: u^2 (u < 2^26 an integer) or, for
+// half-bin 0, kMom0Scale u (u not truncated), as the low bits of the float64
+// 2^52 + that product: one v_fma_f64, exact for u^2 and rounded to the nearest
+// integer for half-bin 0.  The adds carry the bits of 2^52 along
+// (sum_square_words takes them out).
+constexpr double kMom0Scale = 65536.0;
+constexpr unsigned long long kSquareBits = 0x433ull << 52;  // the bits of 2^52
+__device__ __forceinline__ unsigned long long square_word(float u, bool first) {
+  const double ud = (double)u;
+  return (unsigned long long)__double_as_longlong(fma(ud, first ? kMom0Scale : ud, 0x1p52));
+}
+
 // A probability already scaled by 2^m (p in [0, 2^m] or NaN; m = 30 for
 // hard binning, the soft moments' scale otherwise) as m-bit fixed point,
 // truncated: v_cvt_u32_f32 rounds toward zero and maps NaN to 0.  At most
@@ -330,6 +352,17 @@ __device__ __forceinline__ float exp_neg(float x) {
   return __uint_as_float(__float_as_uint(v) + (__float_as_uint(t) << 23));
 }
 
+// 1 / (1 + exp(-x)), correctly rounded from the float32 1 + exp(-x): rcp_rn is
+// the IEEE reciprocal there (its two steps do not depend on the exponent while
+// nothing underflows), in three instructions instead of a division's ten.
+// From 2^126 on (x below -87.3) the quotient is subnormal and v_rcp_f32 gives it
+// within an ulp of 2^-149, 0 for an infinite divisor.
+__device__ __forceinline__ float sigmoid(float x) {
+  const float b = 1.0f + expf(-x);
+  const float y = rcp_rn(b);
+  return b < 0x1p126f ? y : __builtin_amdgcn_rcpf(b);
+}
+
 // In place: logits -> probabilities.  Softmax follows torch.softmax: max over
 // channels, e_c = exp(x_c - max), s = sequential sum over c, p_c = e_c / s
 // (IEEE quotient), with exp_neg.  Sigmoid: 1 / (1 + exp(-x)).
@@ -354,7 +387,7 @@ __device__ __forceinline__ void activate(float (&x)[CMAX], int nc, int act) {
   } else if (act == kActSigmoid) {
 #pragma unroll
     for (int c = 0; c < CMAX; ++c)
-      if (EXACT || c < nc) x[c] = 1.0f / (1.0f + expf(-x[c]));
+      if (EXACT || c < nc) x[c] = sigmoid(x[c]);
   }
 }
 
@@ -530,17 +563,21 @@ struct TableRegs {
     }
   }
   // bscale: a power of two the bucket table is multiplied by (exact)
+  // below: store each edge's predecessor instead (the edges are positive and
+  // normal), so that edge' < p is edge <= p: the right convention with the
+  // left one's comparison
   __device__ __forceinline__ void store(float* lds, const float* btab, const float* rtab, int n,
-                                        int nrepl, int nt, float bscale = 1.0f) const {
+                                        int nrepl, int nt, float bscale = 1.0f, int below = 0) const {
+    auto edge = [&](float v) { return __uint_as_float(__float_as_uint(v) - (uint32_t)below) * bscale; };
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       const int i = (int)threadIdx.x + u * nt;
-      if (i < n + 2) lds[i] = i == 0 ? -__builtin_inff() : (i <= n ? b[u] * bscale : __builtin_inff());
+      if (i < n + 2) lds[i] = i == 0 ? -__builtin_inff() : (i <= n ? edge(b[u]) : __builtin_inff());
       if (i < nrepl) lds[n + 2 + i] = r[u];
     }
     // tables longer than 2 x nt entries
     for (int i = (int)threadIdx.x + 2 * nt; i < n + 2; i += nt)
-      lds[i] = i == n + 1 ? __builtin_inff() : btab[i - 1] * bscale;
+      lds[i] = i == n + 1 ? __builtin_inff() : edge(btab[i - 1]);
     for (int i = (int)threadIdx.x + 2 * nt; i < nrepl; i += nt) lds[n + 2 + i] = rtab[i];
   }
 };
@@ -594,6 +631,8 @@ struct Hist {
   long long* g;           // soft: sum of weight * y                    [CK][R]
   unsigned long long* m2; // moments: sum u^2                           [2CK][R]
   unsigned long long* mg; // moments: sum u over the labelled voxels    [2CK][R]
+  long long* gf;          // moments with per-channel targets: sum of weight * y over
+                          // the targets that are neither 0 nor 1       [CK][R]
 };
 
 // Adds NV voxels (logits xv, labels lab or targets yv) into the histograms.
@@ -780,14 +819,14 @@ __device__ __forceinline__ void zero_sums(unsigned long long* fb, int NV, int re
 // f, coef, jac (one wave per row).  It leaves its final sums zero and returns
 // (in wave 0, unless the reduction is "none") the sum of its rows'
 // per-class errors, in wave_sum's fixed order.
-template <bool SOFT, bool MOM>
+template <bool SOFT, int MOM>
 __device__ __forceinline__ float epilogue(const FwdParams& P, unsigned char* hist,
                                           const float* repl, int CK, int CL, int b0, int nb) {
   const int tid = threadIdx.x;
   const int K = P.K;
-  const int NV = fin_values(CK, MOM, P.packed != 0);
+  const int NV = fin_values(CK, MOM != 0, P.packed != 0, MOM == kMomExactTargets);
   const int reps = P.reps;
-  const EpiLayout L = epi_layout(CK, CL, nb, MOM);
+  const EpiLayout L = epi_layout(CK, CL, nb, MOM != 0);
   const int NB = nb * CK;  // bins of this epilogue
   float* sd = reinterpret_cast<float*>(hist);
   float* sw = sd + NB;
@@ -798,7 +837,19 @@ __device__ __forceinline__ float epilogue(const FwdParams& P, unsigned char* his
   const int64_t BCK = (int64_t)P.B * CK;
   const double dscale = 1.0 / 1073741824.0;  // W and G of the unpacked sums
   const double pscale = P.pscale;             // the sums of p (hard)
+  // sums of the fractional targets of item i (per-channel targets only)
+  auto frac_sum = [&](int i) -> long long {
+    const int bb = nb == 1 ? 0 : i / CK;
+    unsigned long long* fb = P.fin + (int64_t)(b0 + bb) * reps * NV + 10 * CK;
+    long long v[1];
+    load_sums<1>(fb, NV, reps, CK, i - bb * CK, v);
+    zero_sums<1>(fb, NV, reps, CK, i - bb * CK);
+    return v[0];
+  };
+  long long frac0 = 0;  // this thread's first bin, in flight with the moments
   if constexpr (MOM) {
+    if constexpr (MOM == kMomExactTargets)
+      if (tid < NB) frac0 = frac_sum(tid);
     // per half-bin: the five moments (every replica in flight at once), then
     // its six contributions
     const int H2 = 2 * CK;
@@ -812,9 +863,18 @@ __device__ __forceinline__ float epilogue(const FwdParams& P, unsigned char* his
       const int hh = th % (2 * K);
       const double mscale = (double)P.misc;
       const double L = (double)((long long)hh * P.mw) * mscale;
-      moment_terms((double)m[0], (double)m[1], (double)m[2] * mscale,
-                   (double)m[3] * (mscale * mscale * (double)(1ll << P.mshift)),
-                   (double)m[4] * mscale, L, (double)repl[hh], (double)repl[hh + 2], terms + 6 * t);
+      double v1 = (double)m[2] * mscale;
+      double v2 = (double)m[3] * (mscale * mscale * (double)(1ll << P.mshift));
+      if constexpr (MOM >= kMomExact) {
+        // half-bin 0: m[3] is the sum of p itself; both shares of V2 go to bin
+        // 0 and cancel
+        if (hh == 0) {
+          v1 = (double)m[3] * (mscale * (1.0 / kMom0Scale) * (double)(1ll << P.mshift0));
+          v2 = 0.0;
+        }
+      }
+      moment_terms((double)m[0], (double)m[1], v1, v2, (double)m[4] * mscale, L, (double)repl[hh],
+                   (double)repl[hh + 2], terms + 6 * t);
     }
     __syncthreads();
     fast_stamp(P, kTlEpiTerms);
@@ -846,6 +906,7 @@ __device__ __forceinline__ float epilogue(const FwdParams& P, unsigned char* his
           Gd += tb[6 * hh + 5];
         }
       }
+      if constexpr (MOM == kMomExactTargets) Gd += (double)(i == tid ? frac0 : frac_sum(i)) * P.sscale;
     } else if (P.packed) {
       // W << 32 | G (unsigned: W may reach 2^31), then the sum of p
       zero_sums<2>(fb_of(i), NV, reps, CK, t);
@@ -1104,10 +1165,36 @@ __device__ __forceinline__ long long sum_copies_shifted(const unsigned long long
   return acc;
 }
 
+// Exact moments: the second words of R copies, less the bits of 2^52 that each
+// add carried (square_word: n times, n the copy's packed count; modulo 2^64, as
+// the sum itself stays below 2^62), each rounded to a multiple of 2^sh.
+template <int R, int BATCH = kSumBatch>
+__device__ __forceinline__ long long sum_square_words(const unsigned long long* a,
+                                                      const unsigned long long* m2, int w0, int s,
+                                                      int sh) {
+  constexpr int NB = R < BATCH ? R : BATCH;
+  const unsigned long long half = sh > 0 ? 1ull << (sh - 1) : 0ull;
+  long long acc = 0;
+#pragma unroll 1
+  for (int r0 = 0; r0 < R; r0 += NB) {
+    unsigned long long v[NB], n[NB];
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+      const int at = w0 + ((r0 + j + s) & (R - 1));
+      n[j] = a[at] >> kMomShiftN;
+      v[j] = m2[at];
+    }
+#pragma unroll
+    for (int j = 0; j < NB; ++j) acc += (long long)((v[j] - n[j] * kSquareBits + half) >> sh);
+  }
+  return acc;
+}
+
 // Moments variant: 5 values per half-bin (count, labelled count, sum u,
 // sum u^2 >> mshift, labelled sum u of the offsets u of moment_scale;
-// counts unscaled), fin layout [5][2CK].
-template <int R>
+// counts unscaled), fin layout [5][2CK]; with per-channel targets the CK
+// sums of the fractional ones follow.
+template <int R, int MOM>
 __device__ __forceinline__ void block_moments_r(const FwdParams& P, const Hist& H, int CK,
                                                 unsigned long long* fin) {
   const int chunk = 1 << P.lchunk;
@@ -1116,11 +1203,21 @@ __device__ __forceinline__ void block_moments_r(const FwdParams& P, const Hist& 
     long long m[5] = {0, 0, 0, 0, 0};
     // three arrays: half batches keep the registers of the main loop's
     sum_packed<R, kSumBatch / 2, true>(H.a, t * R, t, chunk, m[0], m[1], m[2]);
-    m[3] = sum_copies_shifted<R, kSumBatch / 2>(H.m2, t * R, t, P.mshift);
+    if constexpr (MOM == kMomQuant)
+      m[3] = sum_copies_shifted<R, kSumBatch / 2>(H.m2, t * R, t, P.mshift);
+    else
+      m[3] = sum_square_words<R, kSumBatch / 2>(H.a, H.m2, t * R, t,
+                                                t % (2 * P.K) == 0 ? P.mshift0 : P.mshift);
     m[4] = sum_copies<R, kSumBatch / 2>(H.mg, t * R, t);
 #pragma unroll
     for (int v = 0; v < 5; ++v)
       if (m[v]) atomicAdd(&fin[v * H2 + t], (unsigned long long)m[v]);
+  }
+  if constexpr (MOM == kMomExactTargets) {
+    for (int t = threadIdx.x; t < CK; t += kThreads) {
+      const long long f = sum_copies<R, kSumBatch / 2>(H.gf, t * R, t);
+      if (f) atomicAdd(&fin[5 * H2 + t], (unsigned long long)f);
+    }
   }
 }
 
@@ -1142,7 +1239,8 @@ __device__ __forceinline__ void block_sums_r(const FwdParams& P, const Hist& H, 
         continue;
       }
       s0 = n << kFrac;
-      s2 = sum_copies<R>(H.g1, t * R, t);
+      // targets equal to 1 are counted in the packed word (wide kernels)
+      s2 = sum_copies<R>(H.g1, t * R, t) + (g << kFrac);
     } else {
       s0 = sum_copies<R>(H.w, t * R, t);
       s1 = sum_copies<R>(H.p, t * R, t);
@@ -1154,33 +1252,18 @@ __device__ __forceinline__ void block_sums_r(const FwdParams& P, const Hist& H, 
   }
 }
 
-// Copies per block are a power of two <= 64.
-#define ACE_SWITCH_COPIES(R_, CALL) \
-  switch (R_) {                     \
-    case 1: CALL(1); break;         \
-    case 2: CALL(2); break;         \
-    case 4: CALL(4); break;         \
-    case 8: CALL(8); break;         \
-    case 16: CALL(16); break;       \
-    case 32: CALL(32); break;       \
-    default: CALL(64); break;       \
+// Copies per block are a power of two of at most MAXR (the largest a kernel's
+// geometry gives).
+template <int MAXR, typename F>
+__device__ __forceinline__ void switch_copies(int copies, const F& f) {
+  if constexpr (MAXR > 1) {
+    if (copies < MAXR) {
+      switch_copies<MAXR / 2>(copies, f);
+      return;
+    }
   }
-
-__device__ __forceinline__ void block_moments(const FwdParams& P, const Hist& H, int CK,
-                                              unsigned long long* fin) {
-#define ACE_MOM(R) block_moments_r<R>(P, H, CK, fin)
-  ACE_SWITCH_COPIES(P.copies, ACE_MOM)
-#undef ACE_MOM
+  f(std::integral_constant<int, MAXR>{});
 }
-
-template <bool SOFT>
-__device__ __forceinline__ void block_sums(const FwdParams& P, const Hist& H, int CK, bool labels,
-                                           unsigned long long* fin) {
-#define ACE_SUMS(R) block_sums_r<R, SOFT>(P, H, CK, labels, fin)
-  ACE_SWITCH_COPIES(P.copies, ACE_SUMS)
-#undef ACE_SUMS
-}
-#undef ACE_SWITCH_COPIES
 
 // ---- end of a forward block.  Adds the block's sums into replica
 // (tile % reps) of batch b's final sums (fixed point: exact and
@@ -1190,17 +1273,20 @@ __device__ __forceinline__ void block_sums(const FwdParams& P, const Hist& H, in
 // block, one round trip sooner) and the last batch epilogue to start (which
 // sums the per-class errors into the loss in a fixed order).  Runs in the
 // block's first kThreads threads.
-template <bool SOFT, bool MOM>
+template <bool SOFT, int MOM, int MAXR>
 __device__ __forceinline__ void fwd_finish(const FwdParams& P, const Hist& H, unsigned char* hist,
                                            const float* repl, int CK, int CL, int b,
                                            int64_t tile, bool labels) {
   const int tid = threadIdx.x;
   unsigned long long* fin =
-      P.fin + ((int64_t)b * P.reps + tile % P.reps) * fin_values(CK, MOM, P.packed != 0);
-  if constexpr (MOM)
-    block_moments(P, H, CK, fin);
-  else
-    block_sums<SOFT>(P, H, CK, labels, fin);
+      P.fin + ((int64_t)b * P.reps + tile % P.reps) * fin_values(CK, MOM != 0, P.packed != 0, MOM == kMomExactTargets);
+  switch_copies<MAXR>(P.copies, [&](auto r) {
+    constexpr int R = decltype(r)::value;
+    if constexpr (MOM)
+      block_moments_r<R, MOM>(P, H, CK, fin);
+    else
+      block_sums_r<R, SOFT>(P, H, CK, labels, fin);
+  });
   __shared__ int s_last;
   wait_own_writes();
   __syncthreads();
@@ -1402,7 +1488,7 @@ __global__ void __launch_bounds__(kThreads) fwd_kernel(const FwdParams P) {
     fwd_accumulate<CMAX, EXACT, 1, SOFT, RIGHT>(P, H, btab, repl, nc, copy, xv, lab, yv, labels);
   }
   __syncthreads();
-  fwd_finish<SOFT, false>(P, H, hist, repl, CK, CL, b, tile, labels);
+  fwd_finish<SOFT, kMomNone, 64>(P, H, hist, repl, CK, CL, b, tile, labels);
 }
 
 // ------------------------------------------------------------ backward
@@ -2049,7 +2135,7 @@ __device__ __forceinline__ void fwd_fast_body(const FwdParams& P, const int64_t 
   // other waves end here (a barrier waits only for waves that have not ended)
   if (tid >= kThreads) return;
   fast_stamp(P, kTlLoop);
-  fwd_finish<SOFT, SOFT>(P, H, hist, repl, CK, CL, b, tile, true);
+  fwd_finish<SOFT, SOFT ? kMomQuant : kMomNone, 64>(P, H, hist, repl, CK, CL, b, tile, true);
 }
 
 // Soft backward per half-bin: with the exact-arithmetic weights of the
@@ -2388,8 +2474,7 @@ hipError_t launch(Kern kern, long long nblk, size_t lds, hipStream_t s, const Pa
 
 template <typename T, int CMAX, bool EXACT, int VEC, bool SOFT, bool RIGHT>
 hipError_t launch_fwd_t(const Geometry& g, const FwdParams& prm, hipStream_t s) {
-  // the geometry's voxels per lane (tiles, the alignment test behind
-  // vec_ok) must be the kernel's
+  // the geometry's voxels per lane (its tiles) must be the kernel's
   if (g.var.vec != VEC) return hipErrorInvalidConfiguration;
   auto kern = fwd_kernel<T, CMAX, EXACT, VEC, SOFT, RIGHT>;
   int nt = kThreads;

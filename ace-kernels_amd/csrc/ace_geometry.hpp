@@ -57,17 +57,20 @@ inline size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 //   soft moments (softmax + labels): per half-bin (2K per channel) the packed
 //         word (count | label count | sum u), sum u^2 and sum u over the
 //         labelled voxels, u the offset of the quantised p from the
-//         half-bin's base (moment_scale)
+//         half-bin's base
+//         (moment_scale); with per-channel targets one more i64 per bin, the
+//         sum of the weights times the targets that are neither 0 nor 1
 constexpr size_t hist_bytes_per_copy(int ck, bool soft, bool labels, bool moments = false) {
-  return moments ? (size_t)ck * 48 : (soft ? (size_t)ck * 24 : (size_t)ck * (labels ? 8 : 16));
+  return moments ? (size_t)ck * (labels ? 48 : 56) : (soft ? (size_t)ck * 24 : (size_t)ck * (labels ? 8 : 16));
 }
 
 // Final sums per batch index and replica: 3 x C'K (W, P, G per bin); 2 x C'K
 // for hard binning with class labels (W << 32 | G packed in one word, then
 // P); for soft moments 5 x 2C'K (count, label count, sum u, sum u^2 >>
-// shift, sum u over the labelled voxels per half-bin).
-constexpr int fin_values(int ck, bool moments, bool packed = false) {
-  return moments ? 10 * ck : (packed ? 2 * ck : 3 * ck);
+// shift, sum u over the labelled voxels per half-bin), and with per-channel
+// targets (frac) C'K sums of the fractional targets.
+constexpr int fin_values(int ck, bool moments, bool packed = false, bool frac = false) {
+  return moments ? (frac ? 11 : 10) * ck : (packed ? 2 * ck : 3 * ck);
 }
 
 // LDS layout of an epilogue over nb batch indices (byte offsets from the
@@ -130,6 +133,8 @@ struct Geometry {
   Variant var;
   int nt;              // threads per forward block (kThreads, or kFastThreads for the fast kernels)
   bool fast;           // the forward runs a fast (softmax + class labels) kernel
+  bool wide;           // a wide kernel (ace_wide.hpp), forward and backward
+  bool frac;           // soft moments with per-channel targets: fractional targets' own sums
   bool packed;         // hard binning with labels: W and G share one final-sum word
   int C, CL, off, K, ck;
   int64_t B, N;
@@ -151,6 +156,60 @@ struct Geometry {
   size_t off_fin;      // byte offset of the final sums in the workspace
   size_t ws_bytes;     // workspace bytes; all of it starts zero and is left zero
 };
+
+// What follows from a geometry's block size, copies and steps: the block sums'
+// chunks, the tiles, tickets, replicas, LDS and workspace sizes.
+inline void finish_geometry(Geometry& g, bool soft, size_t per_copy) {
+  const int64_t B = g.B, N = g.N;
+  const int K = g.K;
+  const int copies = g.copies, steps = g.steps;
+  const bool moments = g.moments;
+  const int64_t step_vox = (int64_t)g.nt * g.var.vec;
+  const int64_t copy_cap = moments ? kMaxMomCopyCount : kMaxCopyCount;
+  // block sums: a lane adds the packed words of as many copies as keep the
+  // count fields within kMaxCopyCount before decoding them (a copy counts at
+  // most nt / copies lanes x steps x vec voxels)
+  const int64_t copy_vox = (int64_t)(g.nt / copies) * steps * g.var.vec;
+  int chunk = copies;
+  while (chunk > 1 && (!soft || moments) && chunk * copy_vox > copy_cap) chunk /= 2;
+  int lchunk = 0;
+  while ((1 << lchunk) < chunk) ++lchunk;
+  g.lchunk = lchunk;
+  g.tile_vox = step_vox * steps;
+  g.tiles = N > 0 ? cdiv(N, g.tile_vox) : 1;
+  g.nblk = B * g.tiles;
+  // tickets: one counter per batch index when it has at most
+  // kSingleTicketTiles blocks (one device-scope round trip fewer at the end),
+  // else groups of kGroupTiles blocks, then the groups of a batch index; final
+  // sums replicated so that ~kRepTiles blocks share a replica
+  g.gs = g.tiles <= kSingleTicketTiles ? g.tiles : kGroupTiles;
+  g.gpb = cdiv(g.tiles, g.gs);
+  int64_t reps = cdiv(g.tiles, g.nt == kFastThreads ? kRepTilesFast : kRepTiles);
+  g.reps = (int)(reps > kMaxReps ? kMaxReps : reps);
+  const int n = soft ? 2 * K : K;
+  g.tab_floats = align_up((size_t)(n + 2) + (soft ? (size_t)(2 * K + 2) : 0), 4);
+  // the epilogue block reuses the histogram region (epi_layout).  With one
+  // batch index its epilogue block also sums the loss (no loss ticket); with
+  // more, batch epilogues run in parallel blocks (one block doing several
+  // measured slower on MI355X), then the last one sums the loss.
+  const size_t hist = align_up(per_copy * copies, 16);
+  g.epi_all = B == 1 && g.CL <= kMaxEpiRows;
+  const size_t epi = epi_layout(g.ck, g.CL, 1, moments).bytes;
+  const size_t region = hist > epi ? hist : epi;
+  g.lds_fwd = g.tab_floats * 4 + region;
+  // backward: tables + coef (+ d's two parts) + g, then for soft moments
+  // nine values per half-bin from a 16-byte boundary (bwd_fast_body)
+  g.lds_bwd = (align_up(g.tab_floats + (size_t)g.ck * (soft ? 3 : 1) + (size_t)g.CL, 4) +
+               (moments ? 18 * (size_t)g.ck : 0)) * 4;
+  // workspace: ticket counters (groups, batch indices, loss), one loss
+  // partial word per batch index and the final sums; it must start zero and
+  // every call leaves it zero
+  const int64_t counters = B * g.gpb + B + 1;
+  g.off_part = align_up((size_t)counters * kCtrStride * sizeof(int), 256);
+  g.off_fin = align_up(g.off_part + (size_t)B * sizeof(unsigned long long), 256);
+  const size_t fin_bytes = (size_t)B * g.reps * fin_values(g.ck, moments, g.packed, g.frac) * sizeof(unsigned long long);
+  g.ws_bytes = align_up(g.off_fin + fin_bytes, 256);
+}
 
 // Blocks per batch index: aim for ~4 blocks of 256 threads per CU on a
 // 256-CU part (the generic kernels), or one block of 1024 threads per CU (the
@@ -240,49 +299,59 @@ inline Geometry make_geometry(int64_t B, int64_t C, int64_t N, int K,
     if (steps > max_steps) steps = (int)(max_steps > 0 ? max_steps : 1);
   }
   g.steps = steps;
-  // block sums: a lane adds the packed words of as many copies as keep the
-  // count fields within kMaxCopyCount before decoding them (a copy counts at
-  // most nt / copies lanes x steps x vec voxels)
-  const int64_t copy_vox = (int64_t)(g.nt / copies) * steps * g.var.vec;
-  int chunk = copies;
-  while (chunk > 1 && (!soft || moments) && chunk * copy_vox > copy_cap) chunk /= 2;
-  int lchunk = 0;
-  while ((1 << lchunk) < chunk) ++lchunk;
-  g.lchunk = lchunk;
-  g.tile_vox = step_vox * steps;
-  g.tiles = N > 0 ? cdiv(N, g.tile_vox) : 1;
-  g.nblk = B * g.tiles;
-  // tickets: one counter per batch index when it has at most
-  // kSingleTicketTiles blocks (one device-scope round trip fewer at the end),
-  // else groups of kGroupTiles blocks, then the groups of a batch index; final
-  // sums replicated so that ~kRepTiles blocks share a replica
-  g.gs = g.tiles <= kSingleTicketTiles ? g.tiles : kGroupTiles;
-  g.gpb = cdiv(g.tiles, g.gs);
-  int64_t reps = cdiv(g.tiles, g.nt == kFastThreads ? kRepTilesFast : kRepTiles);
-  g.reps = (int)(reps > kMaxReps ? kMaxReps : reps);
-  const int n = soft ? 2 * K : K;
-  g.tab_floats = align_up((size_t)(n + 2) + (soft ? (size_t)(2 * K + 2) : 0), 4);
-  // the epilogue block reuses the histogram region (epi_layout).  With one
-  // batch index its epilogue block also sums the loss (no loss ticket); with
-  // more, batch epilogues run in parallel blocks (one block doing several
-  // measured slower on MI355X), then the last one sums the loss.
-  const size_t hist = align_up(per_copy * copies, 16);
-  g.epi_all = B == 1 && g.CL <= kMaxEpiRows;
-  const size_t epi = epi_layout(g.ck, g.CL, 1, moments).bytes;
-  const size_t region = hist > epi ? hist : epi;
-  g.lds_fwd = g.tab_floats * 4 + region;
-  // backward: tables + coef (+ d's two parts) + g, then for soft moments
-  // nine values per half-bin from a 16-byte boundary (bwd_fast_body)
-  g.lds_bwd = (align_up(g.tab_floats + (size_t)g.ck * (soft ? 3 : 1) + (size_t)g.CL, 4) +
-               (moments ? 18 * (size_t)g.ck : 0)) * 4;
-  // workspace: ticket counters (groups, batch indices, loss), one loss
-  // partial word per batch index and the final sums; it must start zero and
-  // every call leaves it zero
-  const int64_t counters = B * g.gpb + B + 1;
-  g.off_part = align_up((size_t)counters * kCtrStride * sizeof(int), 256);
-  g.off_fin = align_up(g.off_part + (size_t)B * sizeof(unsigned long long), 256);
-  const size_t fin_bytes = (size_t)B * g.reps * fin_values(g.ck, moments, g.packed) * sizeof(unsigned long long);
-  g.ws_bytes = align_up(g.off_fin + fin_bytes, 256);
+  finish_geometry(g, soft, per_copy);
+  return g;
+}
+
+// ---- wide kernels (ace_wide.hpp): any channel count, softmax or sigmoid,
+// class labels or per-channel targets.
+
+// Channel variants of the wide kernels: cmin < C <= cmax run the variant
+// compiled for cmax channels, the channels above C padded.  Up to 6 channels are exact; above, a step of 2 to 16
+// channels bounds the padding to a fifth and the library's size.
+struct WideVariant {
+  int cmin, cmax, vec;
+};
+constexpr WideVariant kWideVariants[] = {
+    {0, 1, 4},   {1, 2, 4},   {2, 3, 2},   {3, 4, 2},   {4, 5, 1},   {5, 6, 1},   {6, 8, 1},   {8, 10, 1},
+    {10, 12, 1}, {12, 14, 1}, {14, 16, 1}, {16, 20, 1}, {20, 24, 1}, {24, 32, 1}, {32, 48, 1}, {48, 64, 1}};
+inline WideVariant wide_variant(int64_t C) {
+  for (const WideVariant& v : kWideVariants)
+    if (C <= v.cmax) return v;
+  return {0, 0, 0};
+}
+constexpr size_t kMaxWideHistLds = 39 * 1024;  // four blocks per CU with their tables
+constexpr int kMaxWideCopies = 8;
+
+inline Geometry make_wide_geometry(int64_t B, int64_t C, int64_t N, int K, bool soft,
+                                   bool include_background, bool labels) {
+  Geometry g{};
+  const WideVariant v = wide_variant(C);
+  g.wide = true;
+  g.moments = soft;
+  g.frac = soft && !labels;
+  g.packed = !soft && labels;
+  g.var = {v.cmax, v.cmin + 1 == v.cmax, v.vec};
+  g.nt = kThreads;
+  g.C = (int)C;
+  g.off = (!include_background && C > 1) ? 1 : 0;
+  g.CL = (int)C - g.off;
+  g.K = K;
+  g.ck = g.CL * K;
+  g.B = B;
+  g.N = N;
+  const size_t per_copy = hist_bytes_per_copy(g.ck, soft, labels, soft);
+  int copies = kMaxWideCopies;
+  while (copies > 1 && per_copy * copies > kMaxWideHistLds) copies /= 2;
+  g.copies = copies;
+  const int64_t step_vox = (int64_t)g.nt * g.var.vec;
+  int64_t steps = cdiv(B * (N > 0 ? N : 1), step_vox * 1024);
+  const int64_t cap = (int64_t)(soft ? kMaxMomCopyCount : kMaxCopyCount) * copies / step_vox;
+  if (steps > cap) steps = cap;
+  if (steps > 64) steps = 64;
+  if (steps < 1) steps = 1;
+  g.steps = (int)steps;
+  finish_geometry(g, soft, per_copy);
   return g;
 }
 

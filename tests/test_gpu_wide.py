@@ -1,0 +1,166 @@
+"""The wide kernels (any channel count, softmax or sigmoid, class labels or
+per-channel targets) against the CPU reference, at the edges of their channel
+variants and of their steps, with fractional targets, right edges, extreme
+logits, and against the generic kernels, which take a call whose workspace
+holds only their sums."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from ace_kernels import ACEConfig, _lib, ace_loss
+from ace_kernels.impls import hip_mi355x as hip
+from gpu_helpers import LOSS_ATOL, LOSS_RTOL, assert_grad_close, run, say, truth64
+from oracle.reference import reference_ace
+
+pytestmark = pytest.mark.gpu
+
+# both ends of the channel variants (a variant's first count pads most)
+CHANNELS = [1, 2, 3, 4, 5, 6, 7, 8, 9, 11, 13, 14, 15, 16, 17, 20, 21, 24, 25, 32, 33, 48, 49, 64]
+
+
+def _check(x, y, cfg) -> None:
+    loss, grad = run("hip_mi355x", x.cuda(), y.cuda(), cfg)
+    leaf = x.clone().requires_grad_(True)
+    ref = reference_ace(leaf, y, cfg)
+    (ref_grad,) = torch.autograd.grad(ref.sum(), leaf)
+    loss64, grad64 = truth64(x, y, cfg)
+    # the float32 reference's own distance from the float64 result on top
+    err = (ref.detach().double() - loss64).abs()
+    assert bool(((loss.cpu().double() - loss64).abs() <= err + LOSS_RTOL * loss64.abs() + LOSS_ATOL).all())
+    few = cfg.binning == "soft" and x[0, 0].numel() < 100 * cfg.num_bins
+    assert_grad_close(grad, ref_grad, x, cfg, rtol=1e-3 if few else 1e-4, truth=grad64)
+
+
+@pytest.mark.parametrize("binning", ["hard", "soft"])
+@pytest.mark.parametrize("channels", CHANNELS)
+def test_labels(binning, channels) -> None:
+    """Softmax with labels (sigmoid with one channel), an odd row past one step."""
+    gen = torch.Generator().manual_seed(channels)
+    x = torch.randn(2, channels, 33, 31, generator=gen) * 2.0
+    one = channels == 1
+    y = torch.randint(0, max(channels, 2), (2, 1, 33, 31), generator=gen)
+    cfg = ACEConfig(binning=binning, num_bins=10, to_onehot_y=not one, include_background=channels % 3 != 0,
+                    activation="sigmoid" if one else "softmax", right=channels % 2 == 0)
+    say(f"wide labels {binning} C={channels}")
+    _check(x, y.float() if one else y, cfg)
+
+
+@pytest.mark.parametrize("binning", ["hard", "soft"])
+@pytest.mark.parametrize("activation", ["softmax", "sigmoid"])
+@pytest.mark.parametrize("channels,fractional", [(1, True), (2, False), (3, True), (4, True), (5, False), (7, True),
+                                                 (17, True), (33, False), (64, True)])
+def test_targets(binning, activation, channels, fractional) -> None:
+    """Per-channel targets, among them values between 0 and 1 (label
+    smoothing), which take sums of their own."""
+    if channels == 1 and activation == "softmax":
+        pytest.skip("softmax over one channel is no activation")
+    gen = torch.Generator().manual_seed(100 + channels)
+    x = torch.randn(2, channels, 1301, generator=gen) * 2.0
+    y = (torch.rand(2, channels, 1301, generator=gen) < 0.3).float()
+    if fractional:
+        mix = torch.rand(y.shape, generator=gen)
+        y = torch.where(mix < 0.3, mix, y)
+    cfg = ACEConfig(binning=binning, num_bins=12, activation=activation, include_background=channels % 2 == 1)
+    say(f"wide targets {binning} {activation} C={channels} fractional={fractional}")
+    _check(x, y, cfg)
+
+
+@pytest.mark.parametrize("binning", ["hard", "soft"])
+@pytest.mark.parametrize("voxels", [1, 255, 256, 257, 511, 513, 4097])
+def test_steps(binning, voxels) -> None:
+    """Rows that end inside the first step, at its edge, one past it."""
+    gen = torch.Generator().manual_seed(voxels)
+    x = torch.randn(1, 6, voxels, generator=gen)
+    y = torch.randint(0, 6, (1, 1, voxels), generator=gen)
+    cfg = ACEConfig(binning=binning, num_bins=3, to_onehot_y=True)
+    say(f"wide steps {binning} N={voxels}")
+    _check(x, y, cfg)
+
+
+@pytest.mark.parametrize("binning", ["hard", "soft"])
+@pytest.mark.parametrize("channels", [5, 9])
+def test_extreme_logits(binning, channels) -> None:
+    """Voxels with infinite, NaN or very large logits leave every other voxel's
+    gradient as it is without them, up to the sums they count in; saturated
+    voxels match the reference."""
+    gen = torch.Generator().manual_seed(3)
+    x = torch.randn(1, channels, 2000, generator=gen)
+    x[0, :, ::7] *= 400.0
+    y = torch.randint(0, channels, (1, 1, 2000), generator=gen)
+    cfg = ACEConfig(binning=binning, num_bins=10, to_onehot_y=True)
+    say(f"wide extreme {binning} C={channels}")
+    _check(x, y, cfg)
+    x[0, 0, 5], x[0, 1, 6], x[0, 2, 7] = float("inf"), float("-inf"), float("nan")
+    loss, grad = run("hip_mi355x", x.cuda(), y.cuda(), cfg)
+    assert bool(torch.isfinite(loss)) and bool(torch.isfinite(grad[0, :, 8:]).all())
+
+
+def _stats(x, y, cfg, ws_bytes):
+    """W, P, G of one forward given ws_bytes of workspace."""
+    pl = hip.make_plan(x, y, cfg)
+    lib, dev = _lib.lib(), x.device
+    b, cl, k = pl.B, pl.CL, pl.K
+    ws = torch.zeros(ws_bytes, dtype=torch.uint8, device=dev)
+    coef, jac, per = (torch.empty(n, dtype=torch.float32, device=dev) for n in (b * cl * k, b * cl, b * cl))
+    d = torch.empty(2 * b * cl * k, dtype=torch.float32, device=dev)
+    loss = torch.empty((), dtype=torch.float32, device=dev)
+    st = torch.empty(3, b, cl, k, dtype=torch.float64, device=dev)
+    rc = lib.ace_forward(x.data_ptr(), pl.dtype_code, pl.target.data_ptr(), pl.target_kind, b, pl.C, pl.N, k,
+                         _lib.SOFT, pl.act, int(pl.include_bg), 1, _lib.RED_MEAN, int(pl.right), 0.01, None,
+                         pl.btab.data_ptr(), pl.rtab.data_ptr(), ws.data_ptr(), ws_bytes, coef.data_ptr(),
+                         d.data_ptr(), jac.data_ptr(), per.data_ptr(), loss.data_ptr(), st.data_ptr(), hip._stream(dev))
+    return rc, loss, st, ws
+
+
+@pytest.mark.parametrize("channels,labels,activation,bins,right", [
+    (5, True, "softmax", 20, False), (5, True, "softmax", 20, True), (8, True, "softmax", 50, False),
+    (3, False, "softmax", 7, False), (4, False, "sigmoid", 20, True), (1, False, "sigmoid", 33, False),
+    (17, True, "softmax", 10, False), (6, False, "softmax", 100, False), (1, False, "sigmoid", 512, False)])
+def test_same_sums_as_the_generic_kernels(channels, labels, activation, bins, right) -> None:
+    """A workspace too small for the moments (ten or eleven words per bin) but
+    large enough for the generic sums (three) selects the generic kernel: both
+    give the same W, P and G to the generic kernel's fixed point (2^-39 a term
+    at this size), and both leave their workspace zero."""
+    gen = torch.Generator().manual_seed(bins)
+    x = (torch.randn(2, channels, 3001, generator=gen) * 2.0).cuda()
+    if labels:
+        y = torch.randint(0, channels, (2, 1, 3001), generator=gen).cuda()
+    else:
+        y = torch.rand(2, channels, 3001, generator=gen)
+        y = torch.where(y < 0.5, (y < 0.2).float(), y).cuda()
+    cfg = ACEConfig(binning="soft", num_bins=bins, activation=activation, to_onehot_y=labels, right=right)
+    say(f"wide vs generic C={channels} labels={labels} {activation} K={bins} right={right}")
+    full = _lib.lib().ace_workspace_bytes(2, channels, 3001, bins, _lib.SOFT, 0, 1, 0 if labels else 1)
+    rc, loss, wide, ws = _stats(x, y, cfg, full)
+    assert rc == 0 and not bool(ws.any())
+    # the generic layout's size: counters and partials, then 3 C'K words a batch index
+    small = full - 2 * 7 * channels * bins * 8
+    rc, loss_g, generic, ws = _stats(x, y, cfg, small)
+    assert rc == 0 and not bool(ws.any())
+    torch.testing.assert_close(wide, generic, rtol=0, atol=3001 * 2.0 ** -39)
+    torch.testing.assert_close(loss, loss_g, rtol=1e-6, atol=1e-7)
+    rc, *_ = _stats(x, y, cfg, 256)
+    assert rc == 3  # ACE_EWORKSPACE
+
+
+def test_noalloc_scratch_limit() -> None:
+    """A problem whose generic sums fit ace_forward_noalloc's 1 MiB and whose
+    moments do not: still accepted, with the sums of ace_forward."""
+    b, c, n, k = 30, 8, 600, 150
+    gen = torch.Generator().manual_seed(9)
+    x = torch.randn(b, c, n, generator=gen).cuda()
+    y = torch.randint(0, c, (b, 1, n), generator=gen).cuda()
+    cfg = ACEConfig(binning="soft", num_bins=k, to_onehot_y=True)
+    lib, dev = _lib.lib(), x.device
+    assert lib.ace_workspace_bytes(b, c, n, k, _lib.SOFT, 0, 1, 0) > 1 << 20
+    pl = hip.make_plan(x, y, cfg)
+    outs = [torch.empty(m, dtype=torch.float32, device=dev) for m in (b * c * k, 2 * b * c * k, b * c, b * c, 1)]
+    say("wide noalloc at the scratch limit")
+    rc = lib.ace_forward_noalloc(x.data_ptr(), 0, pl.target.data_ptr(), 0, b, c, n, k, _lib.SOFT, pl.act, 1, 1,
+                                 _lib.RED_MEAN, 0, 0.01, None, pl.btab.data_ptr(), pl.rtab.data_ptr(),
+                                 *[o.data_ptr() for o in outs], None, hip._stream(dev))
+    assert rc == 0
+    loss = ace_loss(x, y, cfg, impl="hip_mi355x")
+    torch.testing.assert_close(outs[4][0], loss, rtol=1e-6, atol=1e-7)

@@ -1,0 +1,80 @@
+"""Host-checkable parts of the wide kernels (``csrc/ace_wide.hpp``), on the CPU:
+the exact soft moments' fixed point and the launch geometry."""
+
+from __future__ import annotations
+
+import ctypes
+import subprocess
+from pathlib import Path
+
+import pytest
+import torch
+
+from ace_kernels.common import bin_tables
+
+HERE = Path(__file__).resolve().parent
+CSRC = HERE.parent / "ace-kernels_amd" / "csrc"
+MAX_LDS = 160 * 1024
+
+
+@pytest.fixture(scope="module")
+def lib(tmp_path_factory) -> ctypes.CDLL:
+    out = tmp_path_factory.mktemp("wide") / "libwide.so"
+    subprocess.run(["g++", "-O2", "-shared", "-fPIC", "-std=c++17", "-ffp-contract=off", "-mfma", f"-I{CSRC}",
+                    str(HERE / "wide_harness.cpp"), "-o", str(out)], check=True, capture_output=True)
+    lib = ctypes.CDLL(str(out))
+    ll = ctypes.c_longlong
+    lib.check_exact_moments.restype = ll
+    lib.check_exact_moments.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_double,
+                                        ctypes.c_int]
+    lib.wide_geometry.argtypes = [ll, ll, ll, *[ctypes.c_int] * 4, ctypes.POINTER(ll)]
+    lib.exact_shift.argtypes = [ll, ctypes.c_int]
+    return lib
+
+
+def _half_edges(k: int) -> torch.Tensor:
+    return bin_tables(k, True, torch.device("cpu"))[0]
+
+
+@pytest.mark.parametrize("k", [1, 2, 3, 4, 5, 7, 10, 15, 16, 17, 20, 31, 32, 33, 50, 64, 100, 127, 128, 129, 255, 256,
+                               257, 300, 511, 512])
+def test_exact_moments(lib, k) -> None:
+    """The offset of every probability is exact in float32, an integer from
+    half-bin 1 on, and below 1.2 2^24: its square below 2^50.6."""
+    table = _half_edges(k)
+    assert lib.check_exact_moments(table.data_ptr(), k, 64, 4999, 1.2 * 2 ** 24, 0) == 0
+
+
+def test_a_base_with_too_many_bits_fails(lib) -> None:
+    """An odd base: h w is no float32 for the upper half-bins, or p 2^m - h w
+    needs more than 24 bits."""
+    table = _half_edges(20)
+    assert lib.check_exact_moments(table.data_ptr(), 20, 64, 4999, 1.2 * 2 ** 24, 1) > 0
+
+
+def test_shifts(lib) -> None:
+    """A batch index's sums of u^2 (below 1.2^2 2^48) and of half-bin 0's
+    2^16 u (below 2^40) stay inside int64 after their shift."""
+    for bits in range(0, 41):
+        n = (1 << bits) - 1
+        assert n * 1.2 ** 2 * 2 ** 48 / 2 ** lib.exact_shift(n, 0) < 2 ** 63
+        assert n * 2 ** 40 / 2 ** lib.exact_shift(n, 1) < 2 ** 63
+
+
+@pytest.mark.parametrize("soft", [0, 1])
+@pytest.mark.parametrize("labels", [0, 1])
+def test_geometry(lib, soft, labels) -> None:
+    """Every channel count has a variant that holds it; no copy counts more
+    voxels than its field; the tiles cover the row; the hard layout needs no
+    more workspace than the generic kernels' (same final sums)."""
+    out = (ctypes.c_longlong * 9)()
+    for c in range(1, 65):
+        for n in (0, 1, 255, 256, 257, 20001, 128 ** 3):
+            for k in (1, 20, 50, 512):
+                for b, bg in ((1, 1), (3, 0)):
+                    lib.wide_geometry(b, c, n, k, soft, bg, labels, out)
+                    cmax, vec, copies, steps, _, _, tiles, _, count = out
+                    assert c <= cmax <= max(c + 1, 1.46 * c) and vec in (1, 2, 4)
+                    assert copies in (1, 2, 4, 8) and steps >= 1
+                    assert count <= (4095 if soft else 2047), (c, n, k, count)
+                    assert tiles * 256 * vec * steps >= n
