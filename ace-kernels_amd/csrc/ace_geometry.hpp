@@ -22,6 +22,8 @@ constexpr int kRepTilesFast = 64;          // the same for the fast forward's 10
 constexpr int kMaxReps = 4;                // replicas of the final sums per batch index
 constexpr size_t kMaxFastHistLds = 150 * 1024;  // LDS budget of the histogram copies, 1024-thread blocks
 constexpr int kFastCopies = 16;            // histogram copies of a 1024-thread block
+constexpr int kMaxFastCopies = 64;         // the most that a large problem's step count asks for
+constexpr int64_t kFastBlocks = 256;       // 1024-thread blocks of a launch: one per CU
 
 // Channel variants with a compiled kernel: the kernel keeps C logits of VEC
 // voxels in registers.  EXACT variants fix C at compile time; the others
@@ -246,16 +248,28 @@ inline Geometry make_geometry(int64_t B, int64_t C, int64_t N, int K,
   g.packed = !soft && labels;
   const size_t per_copy = hist_bytes_per_copy(g.ck, soft, labels, moments);
   const bool counted = !soft || moments;  // copies count voxels in 11-bit fields
-  // fast forward: 1024-thread blocks (one per CU) with up to kFastCopies
-  // copies, as many as the LDS holds; each copy counts at most kMaxCopyCount
-  // voxels (nt / copies lanes x steps x vec).  When even one vector step per
-  // lane would overflow a copy, the fast kernel runs with 256-thread blocks.
+  // fast forward: 1024-thread blocks (one per CU) with kFastCopies copies, as
+  // many as the LDS holds; each copy counts at most kMaxCopyCount voxels
+  // (nt / copies lanes x steps x vec).  When even one vector step per lane
+  // would overflow a copy, the fast kernel runs with 256-thread blocks.  A
+  // problem that needs more steps per block than the copies can count (above
+  // 7.8 M voxels at 16 copies) takes more copies rather than a few blocks
+  // more than the CUs, whose second round would run alone: 1 x 4 x 8.8 M
+  // voxels in 288 blocks, 32 of them starting after 30 us, took 57 us; in 256
+  // blocks with 32 copies 42 us.
+  const int64_t fast_step_vox = (int64_t)kFastThreads * g.var.vec;
+  const int64_t fast_steps = cdiv(B * (N > 0 ? N : 1), fast_step_vox * kFastBlocks);
   int fast_copies = 0, fast_steps_max = 0;
   if (fast) {
     int c = copies_override > 0 ? copies_override : kFastCopies;
     while (c > 1 && per_copy * c > kMaxFastHistLds) c /= 2;
+    auto most = [&](int copies) {
+      return (int)((int64_t)kMaxCopyCount / ((int64_t)(kFastThreads / copies) * g.var.vec));
+    };
+    if (copies_override <= 0)
+      while (c < kMaxFastCopies && most(c) < fast_steps && per_copy * c * 2 <= kMaxFastHistLds) c *= 2;
     fast_copies = c;
-    fast_steps_max = (int)((int64_t)kMaxCopyCount / ((int64_t)(kFastThreads / c) * g.var.vec));
+    fast_steps_max = most(c);
   }
   g.fast = fast;
   // 1024 threads for hard binning with C <= 4 only: the 16-channel kernel's
@@ -287,10 +301,19 @@ inline Geometry make_geometry(int64_t B, int64_t C, int64_t N, int K,
     // the chip, and on MI355X ~10% of them started a round late) and issue
     // C x K x 3 final-sum atomics per block (cfg 4, C = 16: 52 us at 512
     // blocks vs 57 us at 1024).  Fast kernels: one 1024-thread block per CU.
-    const int64_t target_blocks = g.nt == kFastThreads ? 256 : (C > 8 ? 512 : 1024);
-    steps = (int)cdiv(total, step_vox * target_blocks);
-    if (steps < 1) steps = 1;
-    if (steps > 64) steps = 64;
+    const int64_t target_blocks = g.nt == kFastThreads ? kFastBlocks : (C > 8 ? 512 : 1024);
+    int64_t want = cdiv(total, step_vox * target_blocks);
+    if (g.nt == kFastThreads) {
+      // whole rounds of blocks: when the copies' counts allow too few steps for
+      // one round, and where each batch index's last, partly filled tile would
+      // add a few blocks to it
+      const int64_t rounds = want > fast_steps_max ? cdiv(want, fast_steps_max) : 1;
+      want = cdiv(want, rounds);
+      while (B <= target_blocks && want < fast_steps_max &&
+             B * cdiv(N, step_vox * want) > target_blocks * rounds)
+        ++want;
+    }
+    steps = (int)(want < 1 ? 1 : (want > 64 ? 64 : want));
   }
   const int64_t copy_cap = moments ? kMaxMomCopyCount : kMaxCopyCount;
   if (counted) {
