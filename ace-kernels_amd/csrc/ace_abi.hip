@@ -186,21 +186,23 @@ size_t workspace_size(int64_t batch, int64_t channels, int64_t voxels, int num_b
 
 // The wide kernels' geometry of a problem, g.wide false where they do not serve
 // it: raw probabilities (no activation: values outside [0, 1]), too many soft
-// bins for the moments' fixed point, or an LDS layout that does not fit.  The
-// generic kernels keep those.
+// bins for the moments' fixed point, an LDS layout that does not fit, or rows
+// shorter than a vector.  The generic kernels keep those.
 Geometry wide_geometry(bool soft, bool labels, int act, int64_t batch, int64_t channels,
-                       int64_t voxels, int num_bins, int include_background) {
+                       int64_t voxels, int num_bins, int include_background, int x_dtype,
+                       bool backward = false) {
   Geometry g{};
   if (act == kActNone || channels > kMaxChannels || (soft && num_bins > kExactMaxBins)) return g;
-  g = make_wide_geometry(batch, channels, voxels, num_bins, soft, include_background != 0, labels);
-  g.wide = g.lds_fwd <= kMaxLds && g.lds_bwd <= kMaxLds && g.nblk <= 0x7fffffffLL;
+  g = make_wide_geometry(batch, channels, voxels, num_bins, soft, include_background != 0, labels,
+                         elem_size(x_dtype), backward);
+  g.wide = voxels >= g.var.vec && g.lds_fwd <= kMaxLds && g.lds_bwd <= kMaxLds && g.nblk <= 0x7fffffffLL;
   return g;
 }
 
 size_t wide_workspace_size(int64_t batch, int64_t channels, int64_t voxels, int num_bins, int binning,
-                           int include_background, int target_kind) {
+                           int x_dtype, int include_background, int target_kind) {
   const Geometry g = wide_geometry(binning == ACE_SOFT, target_kind == ACE_TARGET_LABELS_I64, kActSigmoid,
-                                   batch, channels, voxels, num_bins, include_background);
+                                   batch, channels, voxels, num_bins, include_background, x_dtype);
   return g.wide ? g.ws_bytes : 0;
 }
 
@@ -231,14 +233,15 @@ struct ForwardPlan {
   Geometry g;
 };
 ForwardPlan plan_forward(int64_t batch, int64_t channels, int64_t voxels, int num_bins, int binning,
-                         int activation, int include_background, int target_kind, size_t ws_bytes) {
+                         int activation, int include_background, int target_kind, int x_dtype,
+                         size_t ws_bytes) {
   ForwardPlan fp{};
   const bool soft = binning == ACE_SOFT;
   const bool labels = target_kind == ACE_TARGET_LABELS_I64;
   fp.act = (activation == ACE_ACT_SOFTMAX && channels == 1) ? kActNone : activation;
   fp.moments = use_moments(soft, labels, fp.act, batch, channels, voxels, num_bins, include_background);
   if (!fast_forward(soft, labels, fp.act, channels, fp.moments)) {
-    fp.g = wide_geometry(soft, labels, fp.act, batch, channels, voxels, num_bins, include_background);
+    fp.g = wide_geometry(soft, labels, fp.act, batch, channels, voxels, num_bins, include_background, x_dtype);
     if (fp.g.wide && fp.g.ws_bytes <= ws_bytes) {
       fp.moments = soft;
       return fp;
@@ -523,7 +526,7 @@ size_t ace_workspace_bytes(int64_t batch, int64_t channels, int64_t voxels, int 
   if (batch < 1 || channels < 1 || voxels < 0 || num_bins < 1) return 0;
   if (x_dtype == ACE_F64)
     return f64::workspace_bytes(batch, channels, voxels, num_bins, binning, include_background);
-  const size_t wide = wide_workspace_size(batch, channels, voxels, num_bins, binning,
+  const size_t wide = wide_workspace_size(batch, channels, voxels, num_bins, binning, x_dtype,
                                           include_background, target_kind);
   const size_t rest = workspace_size(batch, channels, voxels, num_bins, binning, include_background,
                                      target_kind);
@@ -554,7 +557,7 @@ int ace_forward(const void* x, int x_dtype, const void* target, int target_kind,
   const bool soft = binning == ACE_SOFT;
   const bool labels = target_kind == ACE_TARGET_LABELS_I64;
   const ForwardPlan fp = plan_forward(batch, channels, voxels, num_bins, binning, activation,
-                                      include_background, target_kind, workspace_bytes);
+                                      include_background, target_kind, x_dtype, workspace_bytes);
   if (fp.rc) return fp.rc;
   const Geometry& g = fp.g;
   const int act = fp.act;
@@ -588,7 +591,10 @@ int ace_backward(const void* x, int x_dtype, const void* target, int target_kind
   // their channel counts with any targets (they read none)
   const bool fast = act == kActSoftmax && fast_channels(channels) && (!soft || moments);
   Geometry g{};
-  if (!fast) g = wide_geometry(soft, labels, act, batch, channels, voxels, num_bins, include_background);
+  // (the wide hard gradient, which reads no targets either, runs as with labels)
+  if (!fast)
+    g = wide_geometry(soft, labels || !soft, act, batch, channels, voxels, num_bins, include_background,
+                      x_dtype, true);
   if (!g.wide)
     g = make_geometry(
         batch, channels, voxels, num_bins, soft, include_background != 0, labels,
@@ -746,7 +752,7 @@ int ace_forward_noalloc(const void* x, int x_dtype, const void* target, int targ
   if (!coef || !diff || !jac || !per_class) return ACE_EINVAL;
   if (reduction != ACE_RED_NONE && !loss) return ACE_EINVAL;
   const ForwardPlan fp = plan_forward(batch, channels, voxels, num_bins, binning, activation,
-                                      include_background, target_kind, ACE_NOALLOC_SCRATCH_BYTES);
+                                      include_background, target_kind, x_dtype, ACE_NOALLOC_SCRATCH_BYTES);
   if (fp.rc) return fp.rc;
   // every layout but the wide kernels', which give way where they do not fit
   size_t need = workspace_size(batch, channels, voxels, num_bins, binning, include_background,

@@ -745,6 +745,24 @@ __device__ __forceinline__ int wave_sum(int v) {
          __builtin_amdgcn_readlane(v, 47) + __builtin_amdgcn_readlane(v, 63);
 }
 
+// The block of the problem's grid that hardware block i of n computes: blocks
+// are dispatched to the eight XCDs in turn, so the blocks of one XCD take one
+// contiguous eighth of the tiles.  The backward takes the same eighths, each
+// from its end, which the forward read last.  For the wide kernels and the
+// 16-channel ones (forward / backward us, mapped and not: soft 2 x 5 x 1.4 M
+// 29.0 / 26.2 and 30.6 / 26.8; one-hot soft 2 x 4 x 1.0 M 25.6 / 18.6 and 26.2 /
+// 19.9; hard 1 x 16 x 128^3 43.2 / 44.1 and 43.5 / 45.9); at four channels and
+// fewer it cost (soft bf16 32 x 4 x 512^2 55.0 / 40.1 against 51.0 / 36.0).
+__device__ __forceinline__ int64_t xcd_block(int64_t i, int64_t n) {
+  const uint32_t u = (uint32_t)i, x = u & 7u, q = (uint32_t)n >> 3, r = (uint32_t)n & 7u;
+  return (int64_t)(x * q + min(x, r) + (u >> 3));
+}
+// The same for the backward, each XCD's eighth from its end.
+__device__ __forceinline__ int64_t xcd_block_back(int64_t i, int64_t n) {
+  const uint32_t u = (uint32_t)i, x = u & 7u, q = (uint32_t)n >> 3, r = (uint32_t)n & 7u;
+  return (int64_t)(x * q + min(x, r) + (q + (x < r ? 1u : 0u) - 1u - (u >> 3)));
+}
+
 // Ticket counter i of the workspace (counters are kCtrStride ints apart).
 __device__ __forceinline__ int* counter(const FwdParams& P, int64_t i) {
   return P.ctr + i * kCtrStride;
@@ -1688,10 +1706,37 @@ __device__ __forceinline__ unsigned long long* bin_at(unsigned long long* base, 
                                                ((uint32_t)k << lsh));
 }
 
+// Keeps the loads issued before it ahead of the code after it, from five
+// channels on.  Without it the scheduler moves the next tile's first arithmetic
+// above the loads of the tile after it, or one tile's labels behind the other
+// tile's logits in the prologue; both put a wait for the youngest loads into
+// the loop, and then a single tile is in flight instead of two (1 x 16 x 128^3
+// hard forward: 44.7 -> 43.5 us).  At four channels and fewer the waves cover
+// one tile's latency and the freer order is the faster one (soft 2 x 4 x 128^3:
+// 33.5 / 26.6 us against 35.0 / 28.3 with it).
+template <int C>
+__device__ __forceinline__ void keep_order() {
+  if constexpr (C > 4) __builtin_amdgcn_sched_barrier(0);
+}
+
 // Load source of the pipelined kernels' first two steps when a tile has no
 // full step: 64 bytes of zeros in device memory (read, never used), so that
 // these loads can be issued unconditionally.
 static __device__ __align__(16) unsigned char g_dummy_src[64];
+
+// Element v of a row.  SC: a uniform pointer plus an unsigned 32-bit byte offset,
+// the address form that takes the row from scalar registers (no vector
+// arithmetic per row and access).  Every backward and the 16-channel forward
+// use it (soft bf16 32 x 4 x 512^2 backward: 37.4 -> 36.0 us); in the forward at
+// four channels and fewer the addresses are a few instructions in a loop that
+// waits for its loads, and their other form left the scheduler the better
+// order (hard 2 x 4 x 128^3, a pass: 47.3 us against 49.5).
+template <bool SC, typename T>
+__device__ __forceinline__ T* row_at(T* row, uint32_t v) {
+  if constexpr (!SC) return row + v;
+  using Byte = typename std::conditional<std::is_const<T>::value, const char, char>::type;
+  return reinterpret_cast<T*>(reinterpret_cast<Byte*>(row) + v * (uint32_t)sizeof(T));
+}
 
 template <int C, int VEC>
 struct FastTile {
@@ -1701,21 +1746,22 @@ struct FastTile {
 
 // One tile's logits and labels; NTL: nontemporal loads of the labels (the
 // hard forward: no later kernel of the step reads them, stream_problem).
-template <typename T, int C, int VEC, bool NTL = false>
+template <typename T, int C, int VEC, bool NTL = false, bool SC = (C > 4)>
 __device__ __forceinline__ void fast_load(FastTile<C, VEC>& t, const T* const (&xr)[C],
                                           const long long* lr, uint32_t v, bool with_labels) {
 #pragma unroll
-  for (int c = 0; c < C; ++c) load_vec<T, VEC>(xr[c] + v, t.x[c]);
+  for (int c = 0; c < C; ++c) load_vec<T, VEC>(row_at<SC>(xr[c], v), t.x[c]);
   if (with_labels) {
+    lr = row_at<SC>(lr, v);
     if constexpr (VEC % 2 == 0) {
 #pragma unroll
       for (int j = 0; j < VEC; j += 2) {
         if constexpr (NTL) {
-          const xi64x2 q = __builtin_nontemporal_load(reinterpret_cast<const xi64x2*>(lr + v + j));
+          const xi64x2 q = __builtin_nontemporal_load(reinterpret_cast<const xi64x2*>(lr + j));
           t.lab[j] = q.x;
           t.lab[j + 1] = q.y;
         } else {
-          const xi64x2 q = *reinterpret_cast<const xi64x2*>(lr + v + j);
+          const xi64x2 q = *reinterpret_cast<const xi64x2*>(lr + j);
           t.lab[j] = q.x;
           t.lab[j + 1] = q.y;
         }
@@ -1724,9 +1770,9 @@ __device__ __forceinline__ void fast_load(FastTile<C, VEC>& t, const T* const (&
 #pragma unroll
       for (int j = 0; j < VEC; ++j) {
         if constexpr (NTL)
-          t.lab[j] = __builtin_nontemporal_load(lr + v + j);
+          t.lab[j] = __builtin_nontemporal_load(lr + j);
         else
-          t.lab[j] = lr[v + j];
+          t.lab[j] = lr[j];
       }
     }
   }
@@ -2088,7 +2134,9 @@ __device__ __forceinline__ void fwd_fast_body(const FwdParams& P, const int64_t 
     for (int c = 0; c < C; ++c) px[c] = pipe ? xr[c] : reinterpret_cast<const T*>(g_dummy_src);
     const long long* pl = pipe ? lr_ : reinterpret_cast<const long long*>(g_dummy_src);
     fast_load<T, C, VEC, !SOFT>(ta, px, pl, pipe ? at(0) : 0u, true);
+    keep_order<C>();
     fast_load<T, C, VEC, !SOFT>(tb, px, pl, pipe ? at(1) : 0u, true);
+    keep_order<C>();
   }
   // soft: the bucket table scaled by 2^m like softmax_fixed's probabilities;
   // hard: as given (the exact path's bucket_unit)
@@ -2113,8 +2161,10 @@ __device__ __forceinline__ void fwd_fast_body(const FwdParams& P, const int64_t 
     for (; i + 2 < nsteps; i += 2) {
       fast_accumulate<C, VEC, SOFT, RIGHT, SKIP0>(ta, tab, P, K, lsh, hb, words);
       fast_load<T, C, VEC, !SOFT>(ta, xr, lr_, at(i + 2), true);
+      keep_order<C>();
       fast_accumulate<C, VEC, SOFT, RIGHT, SKIP0>(tb, tab, P, K, lsh, hb, words);
       fast_load<T, C, VEC, !SOFT>(tb, xr, lr_, at(i + 3), true);
+      keep_order<C>();
     }
     fast_accumulate<C, VEC, SOFT, RIGHT, SKIP0>(ta, tab, P, K, lsh, hb, words);
     if (i + 1 < nsteps) fast_accumulate<C, VEC, SOFT, RIGHT, SKIP0>(tb, tab, P, K, lsh, hb, words);
@@ -2291,8 +2341,10 @@ __device__ __forceinline__ void bwd_fast_body(const BwdParams& P, const int64_t 
 #pragma unroll
     for (int c = 0; c < C; ++c) px[c] = pipe ? xr[c] : reinterpret_cast<const T*>(g_dummy_src);
     const long long* pl = pipe ? lr_ : reinterpret_cast<const long long*>(g_dummy_src);
-    fast_load<T, C, VEC>(ta, px, pl, pipe ? at(0) : 0u, SOFT);
-    fast_load<T, C, VEC>(tb, px, pl, pipe ? at(1) : 0u, SOFT);
+    fast_load<T, C, VEC, false, true>(ta, px, pl, pipe ? at(0) : 0u, SOFT);
+    keep_order<C>();
+    fast_load<T, C, VEC, false, true>(tb, px, pl, pipe ? at(1) : 0u, SOFT);
+    keep_order<C>();
   }
   treg.store(tabs, P.btab, P.rtab, n, nrepl, kThreads);
   if (tid < CK) {
@@ -2327,25 +2379,27 @@ __device__ __forceinline__ void bwd_fast_body(const BwdParams& P, const int64_t 
     for (; i + 2 < nsteps; i += 2) {
       fast_backward<C, VEC, SOFT, RIGHT, SKIP0>(ta, tab, sab, scoef, sg, K);
 #pragma unroll
-      for (int c = 0; c < C; ++c) store_dx<T, VEC, STREAM>(dr[c] + at(i), ta.x[c]);
-      fast_load<T, C, VEC>(ta, xr, lr_, at(i + 2), SOFT);
+      for (int c = 0; c < C; ++c) store_dx<T, VEC, STREAM>(row_at<true>(dr[c], at(i)), ta.x[c]);
+      fast_load<T, C, VEC, false, true>(ta, xr, lr_, at(i + 2), SOFT);
+      keep_order<C>();
       fast_backward<C, VEC, SOFT, RIGHT, SKIP0>(tb, tab, sab, scoef, sg, K);
 #pragma unroll
-      for (int c = 0; c < C; ++c) store_dx<T, VEC, STREAM>(dr[c] + at(i + 1), tb.x[c]);
-      fast_load<T, C, VEC>(tb, xr, lr_, at(i + 3), SOFT);
+      for (int c = 0; c < C; ++c) store_dx<T, VEC, STREAM>(row_at<true>(dr[c], at(i + 1)), tb.x[c]);
+      fast_load<T, C, VEC, false, true>(tb, xr, lr_, at(i + 3), SOFT);
+      keep_order<C>();
     }
     fast_backward<C, VEC, SOFT, RIGHT, SKIP0>(ta, tab, sab, scoef, sg, K);
 #pragma unroll
-    for (int c = 0; c < C; ++c) store_dx<T, VEC, STREAM>(dr[c] + at(i), ta.x[c]);
+    for (int c = 0; c < C; ++c) store_dx<T, VEC, STREAM>(row_at<true>(dr[c], at(i)), ta.x[c]);
     if (i + 1 < nsteps) {
       fast_backward<C, VEC, SOFT, RIGHT, SKIP0>(tb, tab, sab, scoef, sg, K);
 #pragma unroll
-      for (int c = 0; c < C; ++c) store_dx<T, VEC, STREAM>(dr[c] + at(i + 1), tb.x[c]);
+      for (int c = 0; c < C; ++c) store_dx<T, VEC, STREAM>(row_at<true>(dr[c], at(i + 1)), tb.x[c]);
     }
   }
   for (int v = nsteps * stride + tid * VEC; v < nfull; v += stride) {
     FastTile<C, VEC> t;
-    fast_load<T, C, VEC>(t, xr, lr_, (uint32_t)v, SOFT);
+    fast_load<T, C, VEC, false, true>(t, xr, lr_, (uint32_t)v, SOFT);
     fast_backward<C, VEC, SOFT, RIGHT, SKIP0>(t, tab, sab, scoef, sg, K);
 #pragma unroll
     for (int c = 0; c < C; ++c) store_dx<T, VEC, STREAM>(dr[c] + v, t.x[c]);
@@ -2377,14 +2431,16 @@ constexpr int bwd_min_waves() {
 template <typename T, int C, int VEC, bool SOFT, bool RIGHT, bool SKIP0>
 __global__ void __launch_bounds__((fast_bound<C, SOFT>())) fwd_kernel_fast(const FwdParams P) {
   extern __shared__ __align__(16) unsigned char smem[];
-  fwd_fast_body<T, C, VEC, SOFT, RIGHT, SKIP0>(P, blockIdx.x, smem);
+  fwd_fast_body<T, C, VEC, SOFT, RIGHT, SKIP0>(P, C > 4 ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x,
+                                               smem);
 }
 // STREAM: the problem's logits, targets and gradient exceed the last-level
 // cache (stream_problem): the gradient is written with nontemporal stores.
 template <typename T, int C, int VEC, bool SOFT, bool RIGHT, bool SKIP0, bool STREAM>
 __global__ void __launch_bounds__(kThreads, (bwd_min_waves<C, SKIP0>())) bwd_kernel_fast(const BwdParams P) {
   extern __shared__ __align__(16) unsigned char smem[];
-  bwd_fast_body<T, C, VEC, SOFT, RIGHT, SKIP0, STREAM>(P, blockIdx.x, smem);
+  bwd_fast_body<T, C, VEC, SOFT, RIGHT, SKIP0, STREAM>(
+      P, C > 4 ? xcd_block_back(blockIdx.x, gridDim.x) : blockIdx.x, smem);
 }
 
 // Several problems of one configuration in one launch (the levels of a

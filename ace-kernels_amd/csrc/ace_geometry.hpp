@@ -330,31 +330,45 @@ inline Geometry make_geometry(int64_t B, int64_t C, int64_t N, int K,
 // class labels or per-channel targets.
 
 // Channel variants of the wide kernels: cmin < C <= cmax run the variant
-// compiled for cmax channels, the channels above C padded.  Up to 6 channels are exact; above, a step of 2 to 16
-// channels bounds the padding to a fifth and the library's size.
+// compiled for cmax channels, the channels above C padded.  Up to 6 channels are exact; above, steps of 2 to 16
+// channels keep the padding mostly below a tenth and bound the library's size.
 struct WideVariant {
-  int cmin, cmax, vec;
+  int cmin, cmax;
 };
-constexpr WideVariant kWideVariants[] = {
-    {0, 1, 4},   {1, 2, 4},   {2, 3, 2},   {3, 4, 2},   {4, 5, 1},   {5, 6, 1},   {6, 8, 1},   {8, 10, 1},
-    {10, 12, 1}, {12, 14, 1}, {14, 16, 1}, {16, 20, 1}, {20, 24, 1}, {24, 32, 1}, {32, 48, 1}, {48, 64, 1}};
+constexpr WideVariant kWideVariants[] = {{0, 1},   {1, 2},   {2, 3},   {3, 4},   {4, 5},   {5, 6},
+                                         {6, 8},   {8, 10},  {10, 12}, {12, 14}, {14, 16}, {16, 18},
+                                         {18, 20}, {20, 22}, {22, 24}, {24, 28}, {28, 32}, {32, 40},
+                                         {40, 48}, {48, 64}};
 inline WideVariant wide_variant(int64_t C) {
   for (const WideVariant& v : kWideVariants)
     if (C <= v.cmax) return v;
-  return {0, 0, 0};
+  return {0, 0};
+}
+// Voxels per lane and step, consecutive in each row.  Forward: one from five
+// channels on -- it needs no wide loads to stream (5.5 TB/s at 14 rows of
+// 4-byte loads), and a second voxel's registers cost occupancy (8 x 21 x 512^2
+// bf16 hard: 52.8 us at one, 56.5 at two; 1 x 8 x 2.1 M float32: 24.0 / 27.6).
+// Backward: two while two tiles in flight fit, for the stores (the same:
+// 61.4 / 57.4 us; 1 x 14 x 2.5 M float32: 57.8 / 53.3).
+constexpr int wide_vec(int cmax, size_t elem, bool labels, bool backward) {
+  if (cmax <= 2) return 4;
+  if (!backward) return cmax <= 4 ? 2 : 1;
+  if (labels) return elem == 2 || cmax <= 16 ? 2 : 1;
+  return cmax <= 8 ? 2 : 1;
 }
 constexpr size_t kMaxWideHistLds = 39 * 1024;  // four blocks per CU with their tables
 constexpr int kMaxWideCopies = 8;
 
 inline Geometry make_wide_geometry(int64_t B, int64_t C, int64_t N, int K, bool soft,
-                                   bool include_background, bool labels) {
+                                   bool include_background, bool labels, size_t elem,
+                                   bool backward) {
   Geometry g{};
   const WideVariant v = wide_variant(C);
   g.wide = true;
   g.moments = soft;
   g.frac = soft && !labels;
   g.packed = !soft && labels;
-  g.var = {v.cmax, v.cmin + 1 == v.cmax, v.vec};
+  g.var = {v.cmax, v.cmin + 1 == v.cmax, wide_vec(v.cmax, elem, labels, backward)};
   g.nt = kThreads;
   g.C = (int)C;
   g.off = (!include_background && C > 1) ? 1 : 0;

@@ -3,8 +3,8 @@
 // and soft binning in the moments layout.  They serve every such call that
 // the fast kernels (softmax, class labels, C in {2, 3, 4, 16}) do not.
 //
-// One voxel per lane and step from five channels on (two or four below), all
-// its channels in registers.  The channel count is a compile-time CMAX with
+// A lane takes one to four voxels a step (wide_vec), one after the other, all
+// channels of a voxel in registers.  The channel count is a compile-time CMAX with
 // the channels C .. CMAX - 1 padded: they repeat the last row (cache hits)
 // and add 0 to the softmax's sum, so the voxel loop has no branch per
 // channel and every load, exponential and table read of a voxel is in flight
@@ -12,14 +12,15 @@
 // are skipped by a uniform branch.  (A guard per channel, as in the generic
 // kernels, makes each channel a serial chain of waits: 970 cycles per
 // (wave, channel) at C = 21 against the ~100 of its arithmetic.)  Kernel times
-// on MI355X, generic -> wide, forward / backward:
-//   hard 8 x 21 x 512^2 bf16          258 / 245 -> 53 / 62 us
-//   hard 1 x 14 x 97 x 159 x 161      105 / 173 -> 59 / 58 us
-//   soft 2 x 5 x 112 x 128 x 96        64 /  59 -> 31 / 26 us
-//   soft 2 x 4 x 112^2 x 80, targets   43 /  29 -> 28 / 21 us
-//   hard 2 x 3 x 128^3, sigmoid        38 /  24 -> 30 / 20 us
-// A large copy takes the first two 30 / 60 and 20 / 36 us.  What is left is
-// issue: ~25 VALU instructions and an exponential per (voxel, channel).
+// on MI355X, generic -> wide, forward / backward, and the time of a large copy's
+// rate (5.1 TB/s) for the bytes:
+//   hard 8 x 21 x 512^2 bf16          258 / 245 -> 47 / 53 us    20 / 34
+//   hard 1 x 14 x 97 x 159 x 161      105 / 173 -> 44 / 61 us    31 / 54
+//   soft 2 x 5 x 112 x 128 x 96        64 /  59 -> 29 / 26 us    15 / 23
+//   soft 2 x 4 x 112^2 x 80, targets   43 /  29 -> 25 / 18 us    13 / 19
+//   hard 2 x 3 x 128^3, sigmoid        38 /  24 -> 30 / 20 us    20 / 20
+// What is left of the forwards is issue (~25-45 VALU instructions and an
+// exponential per value) and the 6-7 us of the cross-block tail.
 //
 // The probabilities and bins are those of the generic kernels to the bit, and
 // so are the hard sums; the soft sums are the exact ones (exact_moment_scale),
@@ -33,42 +34,72 @@ namespace ace {
 // The `right` convention is folded into the bucket table (TableRegs::store),
 // so every comparison here is the left one.
 
-// One step's voxels of a lane.
-template <int C, int VEC, bool LABELS>
-struct WideTile {
-  float x[C][VEC];
-  long long lab[LABELS ? VEC : 1];
-  float y[LABELS ? 1 : C][VEC];
+// VEC consecutive elements of one row as loaded: converting at the load would
+// wait for it there, and 16-bit pairs take half the registers.
+template <typename T, int VEC>
+struct RawRow {
+  static constexpr int kBytes = VEC * (int)sizeof(T);
+  uint32_t w[(kBytes + 3) / 4];
+  __device__ __forceinline__ void load(const T* p, uint32_t bytes) {
+    using R = typename RawVec<kBytes, sizeof(T)>::type;
+    const R raw = *reinterpret_cast<const R*>(reinterpret_cast<const char*>(p) + bytes);
+    w[0] = 0;
+    __builtin_memcpy(w, &raw, kBytes);
+  }
+  __device__ __forceinline__ float get(int j) const {
+    if constexpr (sizeof(T) == 4) return __uint_as_float(w[j]);
+    const uint32_t pair = w[j >> 1];
+    if constexpr (std::is_same<T, __hip_bfloat16>::value) {
+      return __uint_as_float((j & 1) ? pair & 0xffff0000u : pair << 16);
+    } else {
+      const unsigned short half = (unsigned short)((j & 1) ? pair >> 16 : pair);
+      T v;
+      __builtin_memcpy(&v, &half, 2);
+      return to_f32<T>(v);
+    }
+  }
 };
 
-// Rows C .. CMAX - 1 repeat row nc - 1.
+// One step's voxels of a lane.
+template <typename T, int C, int VEC, bool LABELS>
+struct WideTile {
+  RawRow<T, VEC> x[C];
+  long long lab[LABELS ? VEC : 1];
+  RawRow<float, VEC> y[LABELS ? 1 : C];
+};
+
+// The VEC voxels at v - VEC of every row (v at least 1, and the pointers VEC
+// elements before the tile); rows C .. CMAX - 1 repeat row nc - 1.  A row's
+// uniform pointer plus an unsigned 32-bit byte offset is the address form that
+// takes the row from scalar registers: no vector arithmetic per row.
 template <typename T, int C, int CMIN, int VEC, bool LABELS>
-__device__ __forceinline__ void wide_load(WideTile<C, VEC, LABELS>& t, const T* xt,
-                                          const long long* lt, const float* yt, int64_t N,
-                                          uint32_t v, int nc, bool targets) {
+__device__ __forceinline__ void wide_load(WideTile<T, C, VEC, LABELS>& t, const T* xt,
+                                          const long long* lt, const float* yt, int64_t N, uint32_t v,
+                                          int nc, bool targets) {
 #pragma unroll
   for (int c = 0; c < C; ++c) {
-    load_row<T, VEC>(xt + v, t.x[c]);
-    xt += (c + 1 < CMIN + 1 || c + 1 < nc) ? N : 0;
+    t.x[c].load(xt, v * (uint32_t)sizeof(T));
+    xt += (c < CMIN || c + 1 < nc) ? N : 0;
   }
   if (!targets) return;
   if constexpr (LABELS) {
+    const char* lb = reinterpret_cast<const char*>(lt) + v * 8u;
     if constexpr (VEC % 2 == 0) {
 #pragma unroll
       for (int j = 0; j < VEC; j += 2) {
-        const xi64x2 q = *reinterpret_cast<const xi64x2*>(lt + v + j);
+        const xi64x2 q = *reinterpret_cast<const xi64x2*>(lb + 8 * j);
         t.lab[j] = q.x;
         t.lab[j + 1] = q.y;
       }
     } else {
 #pragma unroll
-      for (int j = 0; j < VEC; ++j) t.lab[j] = lt[v + j];
+      for (int j = 0; j < VEC; ++j) t.lab[j] = *reinterpret_cast<const long long*>(lb + 8 * j);
     }
   } else {
 #pragma unroll
     for (int c = 0; c < C; ++c) {
-      load_row<float, VEC>(yt + v, t.y[c]);
-      yt += (c + 1 < CMIN + 1 || c + 1 < nc) ? N : 0;
+      t.y[c].load(yt, v * 4u);
+      yt += (c < CMIN || c + 1 < nc) ? N : 0;
     }
   }
 }
@@ -205,7 +236,7 @@ __global__ void __launch_bounds__(kThreads, (wide_min_waves(C))) fwd_kernel_wide
   const int R = P.copies;
   const int lsh = __builtin_ctz((unsigned)R) + 3;
   const int tid = threadIdx.x;
-  const int64_t blk = blockIdx.x;
+  const int64_t blk = xcd_block(blockIdx.x, gridDim.x);
   const int b = (int)(blk / P.tiles);
   const int64_t tile = blk - (int64_t)b * P.tiles;
   const int nrepl = SOFT ? 2 * K + 2 : 0;
@@ -224,24 +255,26 @@ __global__ void __launch_bounds__(kThreads, (wide_min_waves(C))) fwd_kernel_wide
   const int64_t N = P.N;
   const int64_t t0 = tile * P.tile_vox;
   const int nvox = (int)min(P.tile_vox, N - t0);
-  const T* xt = reinterpret_cast<const T*>(P.x) + (int64_t)b * nc * N + t0;
-  const long long* lt = reinterpret_cast<const long long*>(P.tgt) + (int64_t)b * N + t0;
-  const float* yt = reinterpret_cast<const float*>(P.tgt) + (int64_t)b * nc * N + t0;
-  const int nfull = (VEC == 1 || P.vec_ok) ? nvox / VEC * VEC : 0;
+  const T* xt = reinterpret_cast<const T*>(P.x) + (int64_t)b * nc * N + t0 - VEC;
+  const long long* lt = reinterpret_cast<const long long*>(P.tgt) + (int64_t)b * N + t0 - VEC;
+  const float* yt = reinterpret_cast<const float*>(P.tgt) + (int64_t)b * nc * N + t0 - VEC;
   constexpr int stride = kThreads * VEC;
 
   TableRegs treg;
   treg.load(P.btab, P.rtab, n, nrepl, kThreads);
-  // two tiles in rotation; loads past the end repeat the last vector
-  WideTile<C, VEC, LABELS> ta, tb;
+  // Two tiles in rotation.  A vector that would pass the tile's end moves back
+  // to end there (rows hold at least VEC voxels, and earlier tiles more); its
+  // first voxels then belong to another lane and are skipped.
+  using Tile = WideTile<T, C, VEC, LABELS>;
+  Tile ta, tb;
   const int v0 = tid * VEC;
-  auto load = [&](WideTile<C, VEC, LABELS>& t, int v) {
-    wide_load<T, C, CMIN, VEC, LABELS>(t, xt, lt, yt, N, (uint32_t)min(v, nfull - VEC), nc, true);
+  const int vlast = nvox - VEC;
+  auto load = [&](Tile& t, int v) {
+    wide_load<T, C, CMIN, VEC, LABELS>(t, xt, lt, yt, N, (uint32_t)(min(v, vlast) + VEC), nc, true);
+    keep_order<C>();
   };
-  if (nfull > 0) {
-    load(ta, v0);
-    load(tb, v0 + stride);
-  }
+  load(ta, v0);
+  load(tb, v0 + stride);
   treg.store(tabs, P.btab, P.rtab, n, nrepl, kThreads, 1.0f, P.right);
   {
     unsigned long long* h64 = reinterpret_cast<unsigned long long*>(hist);
@@ -250,40 +283,28 @@ __global__ void __launch_bounds__(kThreads, (wide_min_waves(C))) fwd_kernel_wide
   __syncthreads();
   const float* repl = tabs + n + 2;
   const int copy = tid & (R - 1);
-  auto bin = [&](WideTile<C, VEC, LABELS>& t, int v) {
-    if (v >= nfull) return;
+  auto bin = [&](Tile& t, int v) {
+    if (v >= nvox) return;
+    const int skip = max(v - vlast, 0);
 #pragma unroll
     for (int j = 0; j < VEC; ++j) {
+      if (j < skip) continue;
       float x[C], y[LABELS ? 1 : C];
 #pragma unroll
-      for (int c = 0; c < C; ++c) x[c] = t.x[c][j];
+      for (int c = 0; c < C; ++c) x[c] = t.x[c].get(j);
       if constexpr (!LABELS) {
 #pragma unroll
-        for (int c = 0; c < C; ++c) y[c] = t.y[c][j];
+        for (int c = 0; c < C; ++c) y[c] = t.y[c].get(j);
       }
       wide_accumulate<C, CMIN, SOFT, LABELS>(P, H, tabs, repl, nc, copy, lsh, x,
                                              LABELS ? t.lab[LABELS ? j : 0] : 0, y);
     }
   };
-  for (int v = v0; v - v0 < nfull; v += 2 * stride) {
+  for (int v = v0; v - v0 < nvox; v += 2 * stride) {
     bin(ta, v);
     load(ta, v + 2 * stride);
     bin(tb, v + stride);
     load(tb, v + 3 * stride);
-  }
-  if constexpr (VEC > 1) {
-    for (int v = nfull + tid; v < nvox; v += kThreads) {
-      WideTile<C, 1, LABELS> t;
-      wide_load<T, C, CMIN, 1, LABELS>(t, xt, lt, yt, N, (uint32_t)v, nc, true);
-      float x[C], y[LABELS ? 1 : C];
-#pragma unroll
-      for (int c = 0; c < C; ++c) x[c] = t.x[c][0];
-      if constexpr (!LABELS) {
-#pragma unroll
-        for (int c = 0; c < C; ++c) y[c] = t.y[c][0];
-      }
-      wide_accumulate<C, CMIN, SOFT, LABELS>(P, H, tabs, repl, nc, copy, lsh, x, LABELS ? t.lab[0] : 0, y);
-    }
   }
   __syncthreads();
   fast_stamp(P, kTlLoop);
@@ -346,15 +367,16 @@ __device__ __forceinline__ void wide_backward(const BwdParams& P, const float* t
   }
 }
 
-// A gradient store, nontemporal for streaming problems: one kernel for both
-// (the empty asm keeps the compiler from merging the two stores into one).
-template <typename T, int VEC>
-__device__ __forceinline__ void store_dx_any(T* p, const float (&in)[VEC], int nt) {
-  if (nt) {
-    store_vec_nt<T, VEC>(p, in);
-    asm volatile("");
-  } else {
-    store_vec<T, VEC>(p, in);
+// One vector of every row's gradient.
+template <typename T, int C, int CMIN, int VEC, bool NT>
+__device__ __forceinline__ void wide_store(T* d, uint32_t v, int64_t N, const float (&out)[C][VEC],
+                                           int nc) {
+  const uint32_t bytes = v * (uint32_t)sizeof(T);
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    if (c <= CMIN || c < nc)
+      store_dx<T, VEC, NT>(reinterpret_cast<T*>(reinterpret_cast<char*>(d) + bytes), out[c]);
+    d += N;
   }
 }
 
@@ -369,7 +391,7 @@ __global__ void __launch_bounds__(kThreads, (wide_min_waves(C))) bwd_kernel_wide
   const int CL = nc - off;
   const int CK = CL * K;
   const int tid = threadIdx.x;
-  const int64_t blk = blockIdx.x;
+  const int64_t blk = xcd_block_back(blockIdx.x, gridDim.x);
   const int b = (int)(blk / P.tiles);
   const int64_t tile = blk - (int64_t)b * P.tiles;
   const int nrepl = SOFT ? 2 * K + 2 : 0;
@@ -384,24 +406,26 @@ __global__ void __launch_bounds__(kThreads, (wide_min_waves(C))) bwd_kernel_wide
   const int64_t N = P.N;
   const int64_t t0 = tile * P.tile_vox;
   const int nvox = (int)min(P.tile_vox, N - t0);
-  const T* xt = reinterpret_cast<const T*>(P.x) + (int64_t)b * nc * N + t0;
-  T* dt = reinterpret_cast<T*>(P.dx) + (int64_t)b * nc * N + t0;
-  const long long* lt = reinterpret_cast<const long long*>(P.tgt) + (int64_t)b * N + t0;
-  const float* yt = reinterpret_cast<const float*>(P.tgt) + (int64_t)b * nc * N + t0;
-  const int nfull = (VEC == 1 || P.vec_ok) ? nvox / VEC * VEC : 0;
+  const T* xt = reinterpret_cast<const T*>(P.x) + (int64_t)b * nc * N + t0 - VEC;
+  T* dt = reinterpret_cast<T*>(P.dx) + (int64_t)b * nc * N + t0 - VEC;
+  const long long* lt = reinterpret_cast<const long long*>(P.tgt) + (int64_t)b * N + t0 - VEC;
+  const float* yt = reinterpret_cast<const float*>(P.tgt) + (int64_t)b * nc * N + t0 - VEC;
   constexpr int stride = kThreads * VEC;
 
   TableRegs treg;
   treg.load(P.btab, P.rtab, n, nrepl, kThreads);
-  WideTile<C, VEC, LABELS> ta, tb;
+  // as in the forward; a vector moved back computes its first voxels as their
+  // own lane does and stores the same bits
+  using Tile = WideTile<T, C, VEC, LABELS>;
+  Tile ta, tb;
   const int v0 = tid * VEC;
-  auto load = [&](WideTile<C, VEC, LABELS>& t, int v) {
-    wide_load<T, C, CMIN, VEC, LABELS>(t, xt, lt, yt, N, (uint32_t)min(v, nfull - VEC), nc, SOFT);
+  const int vlast = nvox - VEC;
+  auto load = [&](Tile& t, int v) {
+    wide_load<T, C, CMIN, VEC, LABELS>(t, xt, lt, yt, N, (uint32_t)(min(v, vlast) + VEC), nc, SOFT);
+    keep_order<C>();
   };
-  if (nfull > 0) {
-    load(ta, v0);
-    load(tb, v0 + stride);
-  }
+  load(ta, v0);
+  load(tb, v0 + stride);
   treg.store(tabs, P.btab, P.rtab, n, nrepl, kThreads, 1.0f, P.right);
   const float* cb = P.coef + (int64_t)b * CK;
   const float* db = P.d + (int64_t)b * CK;
@@ -426,53 +450,38 @@ __global__ void __launch_bounds__(kThreads, (wide_min_waves(C))) bwd_kernel_wide
     soft_half_bin_coefficients(sab, tabs, tabs + n + 2, scoef, sdd, sdl, sg, K, CL);
     __syncthreads();
   }
-  auto grad = [&](WideTile<C, VEC, LABELS>& t, int v) {
-    if (v >= nfull) return;
+  auto grad = [&](Tile& t, int v) {
+    if (v >= nvox) return;
+    float out[C][VEC];
 #pragma unroll
     for (int j = 0; j < VEC; ++j) {
       float x[C], y[LABELS ? 1 : C];
 #pragma unroll
-      for (int c = 0; c < C; ++c) x[c] = t.x[c][j];
+      for (int c = 0; c < C; ++c) x[c] = t.x[c].get(j);
       if constexpr (!LABELS) {
 #pragma unroll
-        for (int c = 0; c < C; ++c) y[c] = t.y[c][j];
+        for (int c = 0; c < C; ++c) y[c] = t.y[c].get(j);
       }
       wide_backward<C, CMIN, SOFT, LABELS>(P, tabs, sab, scoef, nc, x, LABELS ? t.lab[LABELS ? j : 0] : 0, y);
 #pragma unroll
-      for (int c = 0; c < C; ++c) t.x[c][j] = x[c];
+      for (int c = 0; c < C; ++c) out[c][j] = x[c];
     }
-    T* d = dt + v;
-#pragma unroll
-    for (int c = 0; c < C; ++c) {
-      if (c <= CMIN || c < nc) store_dx_any<T, VEC>(d, t.x[c], P.stream);
-      d += N;
+    // one kernel for both kinds of store; the empty asm statements keep the
+    // compiler from merging the two branches into plain stores
+    const uint32_t at = (uint32_t)(min(v, vlast) + VEC);
+    if (P.stream) {
+      asm volatile("" ::: "memory");
+      wide_store<T, C, CMIN, VEC, true>(dt, at, N, out, nc);
+      asm volatile("" ::: "memory");
+    } else {
+      wide_store<T, C, CMIN, VEC, false>(dt, at, N, out, nc);
     }
   };
-  for (int v = v0; v - v0 < nfull; v += 2 * stride) {
+  for (int v = v0; v - v0 < nvox; v += 2 * stride) {
     grad(ta, v);
     load(ta, v + 2 * stride);
     grad(tb, v + stride);
     load(tb, v + 3 * stride);
-  }
-  if constexpr (VEC > 1) {
-    for (int v = nfull + tid; v < nvox; v += kThreads) {
-      WideTile<C, 1, LABELS> t;
-      wide_load<T, C, CMIN, 1, LABELS>(t, xt, lt, yt, N, (uint32_t)v, nc, SOFT);
-      float x[C], y[LABELS ? 1 : C];
-#pragma unroll
-      for (int c = 0; c < C; ++c) x[c] = t.x[c][0];
-      if constexpr (!LABELS) {
-#pragma unroll
-        for (int c = 0; c < C; ++c) y[c] = t.y[c][0];
-      }
-      wide_backward<C, CMIN, SOFT, LABELS>(P, tabs, sab, scoef, nc, x, LABELS ? t.lab[0] : 0, y);
-      T* d = dt + v;
-#pragma unroll
-      for (int c = 0; c < C; ++c) {
-        if (c <= CMIN || c < nc) *d = from_f32<T>(x[c]);
-        d += N;
-      }
-    }
   }
 }
 
@@ -493,18 +502,26 @@ hipError_t allow_lds(Kern kern, size_t lds) {
 template <typename T, bool SOFT, int I>
 hipError_t wide_fwd_variant(const Geometry& g, const FwdParams& p, hipStream_t s) {
   constexpr WideVariant v = kWideVariants[I];
-  auto kern = p.tk == kTgtLabels ? fwd_kernel_wide<T, v.cmax, v.cmin, v.vec, SOFT, true>
-                                 : fwd_kernel_wide<T, v.cmax, v.cmin, v.vec, SOFT, false>;
+  constexpr int vl = wide_vec(v.cmax, sizeof(T), true, false);
+  constexpr int vt = wide_vec(v.cmax, sizeof(T), false, false);
+  const bool labels = p.tk == kTgtLabels;
+  if (g.var.vec != (labels ? vl : vt)) return hipErrorInvalidConfiguration;
+  auto kern = labels ? fwd_kernel_wide<T, v.cmax, v.cmin, vl, SOFT, true>
+                     : fwd_kernel_wide<T, v.cmax, v.cmin, vt, SOFT, false>;
   const hipError_t e = allow_lds(kern, g.lds_fwd);
   return e != hipSuccess ? e : launch(kern, g.nblk, g.lds_fwd, s, p);
 }
 template <typename T, bool SOFT, int I>
 hipError_t wide_bwd_variant(const Geometry& g, const BwdParams& p, hipStream_t s) {
   constexpr WideVariant v = kWideVariants[I];
+  constexpr int vl = wide_vec(v.cmax, sizeof(T), true, true);
+  constexpr int vt = wide_vec(v.cmax, sizeof(T), false, true);
   // the hard gradient reads no targets
-  auto kern = bwd_kernel_wide<T, v.cmax, v.cmin, v.vec, SOFT, true>;
+  const bool labels = !SOFT || p.tk == kTgtLabels;
+  if (g.var.vec != (labels ? vl : vt)) return hipErrorInvalidConfiguration;
+  auto kern = bwd_kernel_wide<T, v.cmax, v.cmin, vl, SOFT, true>;
   if constexpr (SOFT)
-    if (p.tk != kTgtLabels) kern = bwd_kernel_wide<T, v.cmax, v.cmin, v.vec, SOFT, false>;
+    if (!labels) kern = bwd_kernel_wide<T, v.cmax, v.cmin, vt, SOFT, false>;
   const hipError_t e = allow_lds(kern, g.lds_bwd);
   return e != hipSuccess ? e : launch(kern, g.nblk, g.lds_bwd, s, p);
 }
@@ -513,7 +530,7 @@ constexpr int kWideCount = (int)(sizeof(kWideVariants) / sizeof(kWideVariants[0]
 template <typename T, bool SOFT, int I = 0>
 hipError_t wide_fwd_switch(const Geometry& g, const FwdParams& p, hipStream_t s) {
   if constexpr (I < kWideCount) {
-    if (kWideVariants[I].cmax == g.var.cmax && kWideVariants[I].vec == g.var.vec)
+    if (kWideVariants[I].cmax == g.var.cmax)
       return wide_fwd_variant<T, SOFT, I>(g, p, s);
     return wide_fwd_switch<T, SOFT, I + 1>(g, p, s);
   } else {
@@ -523,7 +540,7 @@ hipError_t wide_fwd_switch(const Geometry& g, const FwdParams& p, hipStream_t s)
 template <typename T, bool SOFT, int I = 0>
 hipError_t wide_bwd_switch(const Geometry& g, const BwdParams& p, hipStream_t s) {
   if constexpr (I < kWideCount) {
-    if (kWideVariants[I].cmax == g.var.cmax && kWideVariants[I].vec == g.var.vec)
+    if (kWideVariants[I].cmax == g.var.cmax)
       return wide_bwd_variant<T, SOFT, I>(g, p, s);
     return wide_bwd_switch<T, SOFT, I + 1>(g, p, s);
   } else {

@@ -68,7 +68,7 @@ def test_targets(binning, activation, channels, fractional) -> None:
 
 
 @pytest.mark.parametrize("binning", ["hard", "soft"])
-@pytest.mark.parametrize("voxels", [1, 255, 256, 257, 511, 513, 4097])
+@pytest.mark.parametrize("voxels", [1, 2, 3, 255, 256, 257, 511, 512, 513, 515, 1025, 4097])
 def test_steps(binning, voxels) -> None:
     """Rows that end inside the first step, at its edge, one past it."""
     gen = torch.Generator().manual_seed(voxels)

@@ -27,7 +27,7 @@ def lib(tmp_path_factory) -> ctypes.CDLL:
     lib.check_exact_moments.restype = ll
     lib.check_exact_moments.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_double,
                                         ctypes.c_int]
-    lib.wide_geometry.argtypes = [ll, ll, ll, *[ctypes.c_int] * 4, ctypes.POINTER(ll)]
+    lib.wide_geometry.argtypes = [ll, ll, ll, *[ctypes.c_int] * 6, ctypes.POINTER(ll)]
     lib.exact_shift.argtypes = [ll, ctypes.c_int]
     return lib
 
@@ -63,7 +63,9 @@ def test_shifts(lib) -> None:
 
 @pytest.mark.parametrize("soft", [0, 1])
 @pytest.mark.parametrize("labels", [0, 1])
-def test_geometry(lib, soft, labels) -> None:
+@pytest.mark.parametrize("elem", [2, 4])
+@pytest.mark.parametrize("backward", [0, 1])
+def test_geometry(lib, soft, labels, elem, backward) -> None:
     """Every channel count has a variant that holds it; no copy counts more
     voxels than its field; the tiles cover the row; the hard layout needs no
     more workspace than the generic kernels' (same final sums)."""
@@ -72,7 +74,7 @@ def test_geometry(lib, soft, labels) -> None:
         for n in (0, 1, 255, 256, 257, 20001, 128 ** 3):
             for k in (1, 20, 50, 512):
                 for b, bg in ((1, 1), (3, 0)):
-                    lib.wide_geometry(b, c, n, k, soft, bg, labels, out)
+                    lib.wide_geometry(b, c, n, k, soft, bg, labels, elem, backward, out)
                     cmax, vec, copies, steps, _, _, tiles, _, count = out
                     assert c <= cmax <= max(c + 1, 1.46 * c) and vec in (1, 2, 4)
                     assert copies in (1, 2, 4, 8) and steps >= 1

@@ -68,9 +68,10 @@ long long check_exact_moments(const float* table, int num_bins, int width, int s
 }
 
 // out: {cmax, vec, copies, steps, lds_fwd, lds_bwd, tiles, ws_bytes, largest count of a copy}
-void wide_geometry(long long B, long long C, long long N, int K, int soft, int bg, int labels,
-                   long long* out) {
-  const ace::Geometry g = ace::make_wide_geometry(B, C, N, K, soft != 0, bg != 0, labels != 0);
+void wide_geometry(long long B, long long C, long long N, int K, int soft, int bg, int labels, int elem,
+                   int backward, long long* out) {
+  const ace::Geometry g = ace::make_wide_geometry(B, C, N, K, soft != 0, bg != 0, labels != 0,
+                                               (size_t)elem, backward != 0);
   out[0] = g.var.cmax;
   out[1] = g.var.vec;
   out[2] = g.copies;
