@@ -14,8 +14,8 @@
 // (wave, channel) at C = 21 against the ~100 of its arithmetic.)  Kernel times
 // on MI355X, generic -> wide, forward / backward, and the time of a large copy's
 // rate (5.1 TB/s) for the bytes:
-//   hard 8 x 21 x 512^2 bf16          258 / 245 -> 47 / 53 us    20 / 34
-//   hard 1 x 14 x 97 x 159 x 161      105 / 173 -> 44 / 61 us    31 / 54
+//   hard 8 x 21 x 512^2 bf16          258 / 245 -> 46 / 49 us    20 / 34
+//   hard 1 x 14 x 97 x 159 x 161      105 / 173 -> 44 / 58 us    31 / 54
 //   soft 2 x 5 x 112 x 128 x 96        64 /  59 -> 29 / 26 us    15 / 23
 //   soft 2 x 4 x 112^2 x 80, targets   43 /  29 -> 25 / 18 us    13 / 19
 //   hard 2 x 3 x 128^3, sigmoid        38 /  24 -> 30 / 20 us    20 / 20
@@ -68,6 +68,20 @@ struct WideTile {
   RawRow<float, VEC> y[LABELS ? 1 : C];
 };
 
+// The row stride, above 12 channels opaque to the optimiser, so that row
+// pointers are formed with two scalar adds where they are used.  Known to be
+// the same in every step, the pointers of all rows (and of their gradients)
+// were kept across the loop instead, spilled from the scalar registers into
+// vector lanes, and read back with 2-3 vector instructions per row and access
+// (hard 8 x 21 x 512^2 bf16: 47.6 / 53.0 -> 45.7 / 49.4 us).  Up to 12 channels
+// they fit and keeping them is the cheaper way (eval hard 2 x 7 x 0.4 M: 16.6
+// us against 17.4).
+template <int C>
+__device__ __forceinline__ int64_t row_stride(int64_t n) {
+  if constexpr (C > 12) asm volatile("" : "+s"(n));
+  return n;
+}
+
 // The VEC voxels at v - VEC of every row (v at least 1, and the pointers VEC
 // elements before the tile); rows C .. CMAX - 1 repeat row nc - 1.  A row's
 // uniform pointer plus an unsigned 32-bit byte offset is the address form that
@@ -76,6 +90,7 @@ template <typename T, int C, int CMIN, int VEC, bool LABELS>
 __device__ __forceinline__ void wide_load(WideTile<T, C, VEC, LABELS>& t, const T* xt,
                                           const long long* lt, const float* yt, int64_t N, uint32_t v,
                                           int nc, bool targets) {
+  N = row_stride<C>(N);
 #pragma unroll
   for (int c = 0; c < C; ++c) {
     t.x[c].load(xt, v * (uint32_t)sizeof(T));
@@ -372,6 +387,7 @@ template <typename T, int C, int CMIN, int VEC, bool NT>
 __device__ __forceinline__ void wide_store(T* d, uint32_t v, int64_t N, const float (&out)[C][VEC],
                                            int nc) {
   const uint32_t bytes = v * (uint32_t)sizeof(T);
+  N = row_stride<C>(N);
 #pragma unroll
   for (int c = 0; c < C; ++c) {
     if (c <= CMIN || c < nc)
