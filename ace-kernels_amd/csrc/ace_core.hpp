@@ -670,6 +670,9 @@ __device__ __forceinline__ void fwd_accumulate(const FwdParams& P, const Hist& H
 #pragma unroll
       for (int c = 0; c < CMAX; ++c) {
         if (!(EXACT || c < nc) || c < off) continue;
+        // a NaN counts as 0, as in every other forward kernel: the bits of NaN
+        // weights would land in the fixed-point sums of a whole bin
+        p[c] = p[c] == p[c] ? p[c] : 0.0f;
         const SoftW64 w = soft_assign64<RIGHT>(p[c], K, nf, btab, repl);
         const int sl = ((c - off) * K + w.l) * R + copy;
         const int sr = ((c - off) * K + w.r) * R + copy;

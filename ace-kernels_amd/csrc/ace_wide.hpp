@@ -214,8 +214,9 @@ __device__ __forceinline__ void wide_accumulate(const FwdParams& P, const Hist& 
           if (hit) lds_add(reinterpret_cast<unsigned long long*>(ha + at + 2 * dm2), (unsigned long long)u);
           const float t = y[c];
           if (t != 0.0f && t != 1.0f) {
-            // the exact-arithmetic weights of soft_assign64 at half-bin k
-            const double p = (double)x[c];
+            // the exact-arithmetic weights of soft_assign64 at half-bin k, a NaN
+            // as 0 here too (its weights' bits would land in the sums)
+            const double p = (double)fmaxf(x[c], 0.0f);
             const double ld = p - (double)repl[k];
             const double rd = (double)repl[k + 2] - p;
             const double inv = 1.0 / (ld + rd);

@@ -108,10 +108,48 @@ def _stats(x, y, cfg, ws_bytes):
     loss = torch.empty((), dtype=torch.float32, device=dev)
     st = torch.empty(3, b, cl, k, dtype=torch.float64, device=dev)
     rc = lib.ace_forward(x.data_ptr(), pl.dtype_code, pl.target.data_ptr(), pl.target_kind, b, pl.C, pl.N, k,
-                         _lib.SOFT, pl.act, int(pl.include_bg), 1, _lib.RED_MEAN, int(pl.right), 0.01, None,
-                         pl.btab.data_ptr(), pl.rtab.data_ptr(), ws.data_ptr(), ws_bytes, coef.data_ptr(),
+                         _lib.SOFT if pl.soft else _lib.HARD, pl.act, int(pl.include_bg), 1, _lib.RED_MEAN,
+                         int(pl.right), 0.01, None,
+                         pl.btab.data_ptr(), hip._ptr(pl.rtab), ws.data_ptr(), ws_bytes, coef.data_ptr(),
                          d.data_ptr(), jac.data_ptr(), per.data_ptr(), loss.data_ptr(), st.data_ptr(), hip._stream(dev))
     return rc, loss, st, ws
+
+
+@pytest.mark.parametrize("binning", ["hard", "soft"])
+@pytest.mark.parametrize("kind", ["labels", "onehot", "fractional"])
+@pytest.mark.parametrize("channels", [2, 5, 7])
+def test_nan_probabilities(channels, kind, binning) -> None:
+    """A NaN logit under a sigmoid has a NaN probability, which counts as 0:
+    loss, sums and every other voxel's gradient are those of a logit of minus
+    infinity in its place, in the wide kernels and (soft, a workspace of the
+    generic size) in the generic ones."""
+    gen = torch.Generator().manual_seed(channels)
+    x = (torch.randn(2, channels, 1301, generator=gen) * 2.0).cuda()
+    y = torch.randint(0, channels, (2, 1, 1301), generator=gen)
+    if kind != "labels":
+        y = torch.zeros(2, channels, 1301).scatter_(1, y, 1.0)
+    if kind == "fractional":
+        y = y * 0.8 + 0.1
+    y = y.cuda()
+    bad = torch.zeros(x.shape, dtype=torch.bool, device="cuda")
+    bad[0, 0, 5] = bad[0, 1, 700] = bad[1, channels - 1, 1300] = True
+    nan, low = x.masked_fill(bad, float("nan")), x.masked_fill(bad, float("-inf"))
+    cfg = ACEConfig(binning=binning, num_bins=12, activation="sigmoid", to_onehot_y=kind == "labels")
+    say(f"wide NaN {binning} C={channels} {kind}")
+    (loss, grad), (loss_low, grad_low) = (run("hip_mi355x", t, y, cfg) for t in (nan, low))
+    assert torch.equal(loss, loss_low) and torch.equal(grad[~bad], grad_low[~bad])
+    sizes = [1 << 20]
+    if binning == "soft":
+        sizes.append(_generic_soft_bytes(2, channels, 1301, 12, kind == "labels"))
+    for ws_bytes in sizes:
+        (rc, *got), (rc_low, *want) = (_stats(t, y, cfg, ws_bytes)[:3] for t in (nan, low))
+        assert rc == rc_low == 0 and all(torch.equal(a, b) for a, b in zip(got, want)), ws_bytes
+
+
+def _generic_soft_bytes(b, channels, voxels, bins, labels) -> int:
+    """Workspace bytes that hold the generic soft sums and no moments."""
+    full = _lib.lib().ace_workspace_bytes(b, channels, voxels, bins, _lib.SOFT, 0, 1, 0 if labels else 1)
+    return full - b * (7 if labels else 8) * channels * bins * 8 + 256  # (sizes are multiples of 256)
 
 
 @pytest.mark.parametrize("channels,labels,activation,bins,right", [
