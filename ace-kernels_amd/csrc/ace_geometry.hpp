@@ -7,6 +7,7 @@
 
 namespace ace {
 
+constexpr size_t kLdsPerCu = 160 * 1024;   // gfx950
 constexpr int kThreads = 256;           // threads per block (4 wave64); the epilogue's width
 constexpr int kFastThreads = 1024;      // threads per block of the fast forward kernels (16 wave64)
 constexpr int kFrac = 30;               // fixed-point fraction bits of the sums
@@ -346,13 +347,21 @@ inline WideVariant wide_variant(int64_t C) {
 }
 // Voxels per lane and step, consecutive in each row.  Forward: one from five
 // channels on -- it needs no wide loads to stream (5.5 TB/s at 14 rows of
-// 4-byte loads), and a second voxel's registers cost occupancy (8 x 21 x 512^2
-// bf16 hard: 52.8 us at one, 56.5 at two; 1 x 8 x 2.1 M float32: 24.0 / 27.6).
-// Backward: two while two tiles in flight fit, for the stores (the same:
-// 61.4 / 57.4 us; 1 x 14 x 2.5 M float32: 57.8 / 53.3).
-constexpr int wide_vec(int cmax, size_t elem, bool labels, bool backward) {
+// 4-byte loads), and a second voxel's registers cost occupancy (measured on
+// their first versions, one voxel against two: 8 x 21 x 512^2 bf16 hard 52.8 us
+// against 56.5; 1 x 8 x 2.1 M float32 24.0 / 27.6).  Backward: two while two
+// tiles in flight fit, for the stores (first versions: 57.4 us against 61.4 at
+// one; 1 x 14 x 2.5 M float32 53.3 / 57.8).  The soft gradient with labels also
+// holds the labels and its half-bin coefficients: two voxels fit the registers
+// of wide_min_waves up to 12 channels of 4 bytes, and of 2 bytes up to 14 and at
+// 17-20 (fewer waves); elsewhere they spilled 20 to 342 registers (soft, K = 20,
+// two voxels -> one: 1 x 14 x 0.57 M float32 20.6 -> 15.8 us, bf16 1 x 15 x 0.8 M
+// 25.1 -> 21.1, bf16 1 x 24 x 0.5 M 49.1 -> 25.5; where two fit they stay
+// faster, bf16 1 x 20 x 0.6 M 21.5 against 25.9).
+constexpr int wide_vec(int cmax, size_t elem, bool soft, bool labels, bool backward) {
   if (cmax <= 2) return 4;
   if (!backward) return cmax <= 4 ? 2 : 1;
+  if (labels && soft) return cmax <= (elem == 2 ? 14 : 12) || (elem == 2 && cmax > 16 && cmax <= 20) ? 2 : 1;
   if (labels) return elem == 2 || cmax <= 16 ? 2 : 1;
   return cmax <= 8 ? 2 : 1;
 }
@@ -368,7 +377,7 @@ inline Geometry make_wide_geometry(int64_t B, int64_t C, int64_t N, int K, bool 
   g.moments = soft;
   g.frac = soft && !labels;
   g.packed = !soft && labels;
-  g.var = {v.cmax, v.cmin + 1 == v.cmax, wide_vec(v.cmax, elem, labels, backward)};
+  g.var = {v.cmax, v.cmin + 1 == v.cmax, wide_vec(v.cmax, elem, soft, labels, backward)};
   g.nt = kThreads;
   g.C = (int)C;
   g.off = (!include_background && C > 1) ? 1 : 0;
@@ -389,6 +398,23 @@ inline Geometry make_wide_geometry(int64_t B, int64_t C, int64_t N, int K, bool 
   if (steps < 1) steps = 1;
   g.steps = (int)steps;
   finish_geometry(g, soft, per_copy);
+  if (soft && backward) {
+    // whole rounds of blocks: the half-bin coefficients (84 bytes per bin) may
+    // leave room for a few blocks per CU only, and each block forms them anew
+    // (soft 1 x 14 x 143 k float32, K = 50: 560 blocks at two per CU, 48 of them
+    // in a second round, 14.2 us; 280 blocks 11.3; bf16 1 x 20 x 250 k: 22.4 ->
+    // 17.0)
+    const int64_t fit = (int64_t)(kLdsPerCu / g.lds_bwd);
+    const int64_t round = 256 * fit;
+    if (fit > 0 && fit < 4 && g.nblk > round) {
+      const int64_t rounds = g.nblk / round;
+      const int64_t fewer = cdiv(B * cdiv(N, step_vox), round * rounds);
+      if (fewer > steps && fewer <= cap) {
+        g.steps = (int)fewer;
+        finish_geometry(g, soft, per_copy);
+      }
+    }
+  }
   return g;
 }
 

@@ -519,8 +519,8 @@ hipError_t allow_lds(Kern kern, size_t lds) {
 template <typename T, bool SOFT, int I>
 hipError_t wide_fwd_variant(const Geometry& g, const FwdParams& p, hipStream_t s) {
   constexpr WideVariant v = kWideVariants[I];
-  constexpr int vl = wide_vec(v.cmax, sizeof(T), true, false);
-  constexpr int vt = wide_vec(v.cmax, sizeof(T), false, false);
+  constexpr int vl = wide_vec(v.cmax, sizeof(T), SOFT, true, false);
+  constexpr int vt = wide_vec(v.cmax, sizeof(T), SOFT, false, false);
   const bool labels = p.tk == kTgtLabels;
   if (g.var.vec != (labels ? vl : vt)) return hipErrorInvalidConfiguration;
   auto kern = labels ? fwd_kernel_wide<T, v.cmax, v.cmin, vl, SOFT, true>
@@ -531,8 +531,8 @@ hipError_t wide_fwd_variant(const Geometry& g, const FwdParams& p, hipStream_t s
 template <typename T, bool SOFT, int I>
 hipError_t wide_bwd_variant(const Geometry& g, const BwdParams& p, hipStream_t s) {
   constexpr WideVariant v = kWideVariants[I];
-  constexpr int vl = wide_vec(v.cmax, sizeof(T), true, true);
-  constexpr int vt = wide_vec(v.cmax, sizeof(T), false, true);
+  constexpr int vl = wide_vec(v.cmax, sizeof(T), SOFT, true, true);
+  constexpr int vt = wide_vec(v.cmax, sizeof(T), SOFT, false, true);
   // the hard gradient reads no targets
   const bool labels = !SOFT || p.tk == kTgtLabels;
   if (g.var.vec != (labels ? vl : vt)) return hipErrorInvalidConfiguration;

@@ -4,12 +4,15 @@ the exact soft moments' fixed point and the launch geometry."""
 from __future__ import annotations
 
 import ctypes
+import re
+import struct
 import subprocess
 from pathlib import Path
 
 import pytest
 import torch
 
+from ace_kernels import _lib
 from ace_kernels.common import bin_tables
 
 HERE = Path(__file__).resolve().parent
@@ -80,3 +83,60 @@ def test_geometry(lib, soft, labels, elem, backward) -> None:
                     assert copies in (1, 2, 4, 8) and steps >= 1
                     assert count <= (4095 if soft else 2047), (c, n, k, count)
                     assert tiles * 256 * vec * steps >= n
+
+
+@pytest.mark.parametrize("channels,bins,voxels,elem,most", [
+    (14, 50, 143_312, 4, 512), (14, 100, 70_602, 4, 256), (20, 50, 250_047, 2, 512), (24, 50, 83_248, 2, 256),
+    (24, 50, 499_280, 2, 768)])
+def test_soft_backward_whole_rounds(lib, channels, bins, voxels, elem, most) -> None:
+    """The half-bin coefficients leave room for one or two blocks of these
+    soft gradients per CU: their blocks are no few more than a whole number of
+    rounds."""
+    out = (ctypes.c_longlong * 9)()
+    lib.wide_geometry(1, channels, voxels, bins, 1, 1, 1, elem, 1, out)
+    lds, tiles = out[5], out[6]
+    round_ = 256 * (160 * 1024 // lds)
+    assert round_ in (256, 512) and tiles <= most and most % round_ == 0
+
+
+def _spills(path: Path) -> dict:
+    """Kernel name -> vector registers spilled, from the metadata of the code
+    objects in the built library."""
+    msgpack = pytest.importorskip("msgpack")
+    data = path.read_bytes()
+    magic, out, at = b"__CLANG_OFFLOAD_BUNDLE__", {}, 0
+    while (at := data.find(magic, at)) >= 0:
+        pos = at + 32
+        for _ in range(struct.unpack_from("<Q", data, at + 24)[0]):
+            off, size, length = struct.unpack_from("<QQQ", data, pos)
+            target = data[pos + 24:pos + 24 + length]
+            pos += 24 + length
+            if b"gfx950" not in target or not size:
+                continue
+            elf = data[at + off:at + off + size]
+            table, = struct.unpack_from("<Q", elf, 0x28)
+            entry, count = struct.unpack_from("<HH", elf, 0x3a)
+            for h in range(table, table + entry * count, entry):
+                if struct.unpack_from("<I", elf, h + 4)[0] != 7:  # SHT_NOTE
+                    continue
+                note, = struct.unpack_from("<Q", elf, h + 0x18)
+                name, desc, kind = struct.unpack_from("<III", elf, note)
+                start = note + 12 + (name + 3) // 4 * 4
+                assert kind == 32  # NT_AMDGPU_METADATA
+                for k in msgpack.unpackb(elf[start:start + desc])["amdhsa.kernels"]:
+                    out[k[".name"]] = k[".vgpr_spill_count"]
+        at += len(magic)
+    return out
+
+
+def test_label_kernels_up_to_24_channels_do_not_spill() -> None:
+    """Two tiles in flight stay in vector registers for class labels, both
+    binnings and directions, but for a handful of registers."""
+    kernel = re.compile(r"(fwd|bwd)_kernel_wideI\w+?Li(\d+)ELi\d+ELi\d+ELb([01])ELb1E")
+    found = 0
+    for name, spilled in _spills(_lib.LIB_PATH).items():
+        m = kernel.search(name)
+        if m and int(m.group(2)) <= 24:
+            found += 1
+            assert spilled <= 16, (name, spilled)
+    assert found == 15 * 3 * 2 * 2  # variants x element types x binnings x directions
