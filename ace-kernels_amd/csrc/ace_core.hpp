@@ -352,15 +352,19 @@ __device__ __forceinline__ float exp_neg(float x) {
   return __uint_as_float(__float_as_uint(v) + (__float_as_uint(t) << 23));
 }
 
-// 1 / (1 + exp(-x)), correctly rounded from the float32 1 + exp(-x): rcp_rn is
-// the IEEE reciprocal there (its two steps do not depend on the exponent while
-// nothing underflows), in three instructions instead of a division's ten.
-// From 2^126 on (x below -87.3) the quotient is subnormal and v_rcp_f32 gives it
-// within an ulp of 2^-149, 0 for an infinite divisor.
+// 1 / (1 + exp(-x)): the IEEE quotient of the float32 1 + exp(-x), in six
+// instructions instead of a division's ten.  v_rcp_f32 flushes the subnormal
+// quotients of divisors from 2^126 on (x below -87.3) to 0, so it takes the
+// reciprocal of b / 4, which is scaled back (both exact while the quotient is
+// normal); rcp_rn's two steps then correct it as there, with b held finite, so
+// that 1 / inf is 0.  Over all 2^24 subnormal quotients, with v_rcp_f32 an ulp
+// off either way, at most 6 come out one unit of 2^-149 beside the IEEE
+// quotient.
 __device__ __forceinline__ float sigmoid(float x) {
   const float b = 1.0f + expf(-x);
-  const float y = rcp_rn(b);
-  return b < 0x1p126f ? y : __builtin_amdgcn_rcpf(b);
+  const float y = __builtin_amdgcn_rcpf(b * 0.25f) * 0.25f;
+  const float e = fmaf(-fminf(b, 0x1.fffffep127f), y, 1.0f);
+  return fmaf(e, y, y);
 }
 
 // In place: logits -> probabilities.  Softmax follows torch.softmax: max over

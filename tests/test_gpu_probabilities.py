@@ -119,3 +119,21 @@ def test_probabilities_are_a_softmax() -> None:
         torch.testing.assert_close(pk.sum(1), torch.ones_like(pk.sum(1)), rtol=0, atol=1e-6)
         ps = kernel_probs(x, ACEConfig(activation="sigmoid"))
         torch.testing.assert_close(ps, torch.sigmoid(x.float()), rtol=5e-7, atol=1e-30)
+
+
+def test_sigmoid_of_very_negative_logits() -> None:
+    """1 / (1 + exp(-x)) down to its smallest values: below x = -87.3 it is
+    subnormal, and 0 only from -88.73, where exp(-x) overflows.  Against float64:
+    an ulp of exp and half an ulp of the sum and of the quotient (2^-22 in all),
+    and half of 2^-149 where the quotient is subnormal."""
+    low = torch.linspace(-88.7, -86.5, 40001)
+    # beside an ordinary channel, in the last of the channels, and alone
+    x = torch.stack([low, torch.randn(low.shape, generator=torch.Generator().manual_seed(1)), low.flip(0)])[None]
+    say("probabilities: sigmoid near its smallest values")
+    for t in (x, x[:, :1]):
+        p = kernel_probs(t, ACEConfig(activation="sigmoid")).double()
+        exact = torch.sigmoid(t.double())
+        assert bool(((p - exact).abs() <= 2.0 ** -22 * exact + 2.0 ** -150).all())
+    ends = torch.tensor([-89.0, -1e30, -float("inf"), float("inf"), 1e30, 0.0])[None, None]
+    got = kernel_probs(ends, ACEConfig(activation="sigmoid"))[0, 0]
+    assert got.tolist() == [0.0, 0.0, 0.0, 1.0, 1.0, 0.5]
