@@ -225,7 +225,8 @@ int bwd_steps(bool soft, bool labels, int act, int64_t batch, int64_t channels, 
 // launched: the geometry of the kernel the launcher will pick, within the
 // LDS and the grid's limits.  A wide kernel whose final sums do not fit in
 // ws_bytes of workspace (the moments hold ten words per bin, the generic soft
-// sums three) leaves the call to the generic kernel.
+// sums three) leaves the call to the generic kernel, and so does the soft one
+// where that is faster (wide_soft_forward_pays).
 struct ForwardPlan {
   int rc;
   int act;
@@ -240,16 +241,18 @@ ForwardPlan plan_forward(int64_t batch, int64_t channels, int64_t voxels, int nu
   const bool labels = target_kind == ACE_TARGET_LABELS_I64;
   fp.act = (activation == ACE_ACT_SOFTMAX && channels == 1) ? kActNone : activation;
   fp.moments = use_moments(soft, labels, fp.act, batch, channels, voxels, num_bins, include_background);
-  if (!fast_forward(soft, labels, fp.act, channels, fp.moments)) {
-    fp.g = wide_geometry(soft, labels, fp.act, batch, channels, voxels, num_bins, include_background, x_dtype);
-    if (fp.g.wide && fp.g.ws_bytes <= ws_bytes) {
-      fp.moments = soft;
-      return fp;
-    }
-  }
   fp.g = forward_geometry(batch, channels, voxels, num_bins, soft, include_background, labels, fp.act,
                           fp.moments);
   fp.rc = (fp.g.lds_fwd > kMaxLds || fp.g.nblk > 0x7fffffffLL) ? ACE_EUNSUPPORTED : ACE_OK;
+  if (!fast_forward(soft, labels, fp.act, channels, fp.moments)) {
+    const Geometry w =
+        wide_geometry(soft, labels, fp.act, batch, channels, voxels, num_bins, include_background, x_dtype);
+    if (w.wide && w.ws_bytes <= ws_bytes && (!soft || fp.rc || wide_soft_forward_pays(w, fp.g, labels))) {
+      fp.g = w;
+      fp.moments = soft;
+      fp.rc = ACE_OK;
+    }
+  }
   return fp;
 }
 

@@ -418,4 +418,35 @@ inline Geometry make_wide_geometry(int64_t B, int64_t C, int64_t N, int K, bool 
   return g;
 }
 
+// Whether the wide kernel (geometry w) is the faster forward of a soft problem
+// that the generic kernel (geometry g) serves too.  It bins a voxel in a third
+// to a half of the time, but adds 10 or 11 final-sum words per bin and block
+// (g: 3), and its epilogue forms six float64 terms per half-bin.  The
+// difference of their times in us,
+//   fixed + 0.024 C'K + 1.05e-5 (words x blocks, wide - generic) - gain x 1e-6 x values,
+// with fixed and gain by the generic kernel's variant (gain 1.6 and 2.4 times
+// where its lanes share two or one histogram copies, whose adds collide), was
+// fitted to 1500 sizes on MI355X (1-24 channels, 5-100 bins, 600 to 16 M
+// voxels): choosing by its sign is within 0.3 % of the faster kernel on average,
+// the wide one alone 6 % (at most 2.0 x: sigmoid 1 x 4 x 0.5 M, K = 100: 18.6 us
+// generic, 37.0 wide; labels 1 x 8 x 250 k, K = 50: 24.5 / 35.8; 1 x 8 x 2 M,
+// K = 50: 96.4 / 53.0).  Above 16 channels the wide kernel is the faster one at
+// nearly every size.
+struct SoftForwardCost {
+  int cmax;
+  double fixed, gain;
+};
+constexpr SoftForwardCost kSoftLabelsCost[] = {{8, -6.7, 3.1}, {16, -10.8, 8.8}};
+constexpr SoftForwardCost kSoftTargetsCost[] = {{1, -0.4, 3.5}, {4, -7.3, 2.0}, {8, -3.6, 3.3}, {16, -6.8, 4.2}};
+inline bool wide_soft_forward_pays(const Geometry& w, const Geometry& g, bool labels) {
+  if (w.C > 16) return true;
+  const SoftForwardCost* cost = labels ? kSoftLabelsCost : kSoftTargetsCost;
+  while (cost->cmax < w.C) ++cost;
+  const double gain = cost->gain * (g.copies == 1 ? 2.4 : (g.copies == 2 ? 1.6 : 1.0));
+  const double words = (double)fin_values(w.ck, true, false, !labels) * (double)w.nblk -
+                       (double)fin_values(g.ck, false) * (double)g.nblk;
+  const double values = (double)w.B * (double)w.N * w.C;
+  return cost->fixed + 0.024 * w.ck + 1.05e-5 * words - gain * 1e-6 * values <= 0.0;
+}
+
 }  // namespace ace

@@ -157,7 +157,8 @@ def _generic_soft_bytes(b, channels, voxels, bins, labels) -> int:
     (3, False, "softmax", 7, False), (4, False, "sigmoid", 20, True), (1, False, "sigmoid", 33, False),
     (17, True, "softmax", 10, False), (6, False, "softmax", 100, False), (1, False, "sigmoid", 512, False)])
 def test_same_sums_as_the_generic_kernels(channels, labels, activation, bins, right) -> None:
-    """A workspace too small for the moments (ten or eleven words per bin) but
+    """(At many bins both sides run the generic kernel, the faster one there.)
+    A workspace too small for the moments (ten or eleven words per bin) but
     large enough for the generic sums (three) selects the generic kernel: both
     give the same W, P and G to the generic kernel's fixed point (2^-39 a term
     at this size), and both leave their workspace zero."""
@@ -181,6 +182,35 @@ def test_same_sums_as_the_generic_kernels(channels, labels, activation, bins, ri
     torch.testing.assert_close(loss, loss_g, rtol=1e-6, atol=1e-7)
     rc, *_ = _stats(x, y, cfg, 256)
     assert rc == 3  # ACE_EWORKSPACE
+
+
+@pytest.mark.parametrize("channels,labels,activation,bins,voxels", [
+    (5, True, "softmax", 50, 1_600_003), (8, True, "softmax", 50, 2_000_001), (14, True, "softmax", 20, 300_007),
+    (1, False, "sigmoid", 50, 4_000_001), (4, False, "sigmoid", 100, 4_000_003), (8, False, "softmax", 20, 1_000_003)])
+def test_large_problems_match_the_generic_kernels(channels, labels, activation, bins, voxels) -> None:
+    """As above where many blocks of several steps run and the wide kernel is
+    the faster one: tiles in rotation, copies near their count's limit, and
+    replicas of the final sums."""
+    gen = torch.Generator(device="cuda").manual_seed(bins)
+    x = torch.randn(1, channels, voxels, generator=gen, device="cuda") * 2.0
+    if labels:
+        y = torch.randint(0, channels, (1, 1, voxels), generator=gen, device="cuda")
+    else:
+        y = torch.rand(1, channels, voxels, generator=gen, device="cuda")
+        y = torch.where(y < 0.5, (y < 0.2).float(), y)
+    cfg = ACEConfig(binning="soft", num_bins=bins, activation=activation, to_onehot_y=labels)
+    say(f"wide vs generic C={channels} labels={labels} {activation} K={bins} N={voxels}")
+    full = _lib.lib().ace_workspace_bytes(1, channels, voxels, bins, _lib.SOFT, 0, 1, 0 if labels else 1)
+    rc, loss, wide, ws = _stats(x, y, cfg, full)
+    assert rc == 0 and not bool(ws.any())
+    rc, loss_g, generic, ws = _stats(x, y, cfg, _generic_soft_bytes(1, channels, voxels, bins, labels))
+    assert rc == 0 and not bool(ws.any())
+    # the generic kernels round each of a voxel's terms to half a unit of their
+    # fixed point: 2^-41, coarser for more than 2^19 voxels (soft_frac)
+    unit = 2.0 ** -min(40, 60 - voxels.bit_length())
+    assert not torch.equal(wide, generic)  # two kernels
+    torch.testing.assert_close(wide, generic, rtol=0, atol=voxels * unit)
+    torch.testing.assert_close(loss, loss_g, rtol=1e-6, atol=1e-7)
 
 
 def test_noalloc_scratch_limit() -> None:

@@ -32,6 +32,7 @@ def lib(tmp_path_factory) -> ctypes.CDLL:
                                         ctypes.c_int]
     lib.wide_geometry.argtypes = [ll, ll, ll, *[ctypes.c_int] * 6, ctypes.POINTER(ll)]
     lib.exact_shift.argtypes = [ll, ctypes.c_int]
+    lib.soft_forward_wide.argtypes = [ll, ll, ll, *[ctypes.c_int] * 3]
     return lib
 
 
@@ -97,6 +98,38 @@ def test_soft_backward_whole_rounds(lib, channels, bins, voxels, elem, most) -> 
     lds, tiles = out[5], out[6]
     round_ = 256 * (160 * 1024 // lds)
     assert round_ in (256, 512) and tiles <= most and most % round_ == 0
+
+
+# measured on MI355X: (batch, channels, voxels, bins, labels), the kernel that was
+# faster by a tenth or more
+GENERIC_FASTER = [
+    (1, 5, 198_476, 50, 1), (1, 8, 250_047, 32, 1), (1, 8, 250_047, 50, 1), (1, 8, 499_280, 100, 1),
+    (16, 8, 8000, 50, 1), (1, 10, 198_476, 50, 1), (1, 12, 83_248, 50, 1), (1, 12, 166_375, 100, 1),
+    (1, 3, 666_072, 100, 0), (1, 4, 499_280, 100, 0), (1, 5, 198_476, 50, 0), (2, 8, 29_791, 50, 0),
+    (1, 8, 250_047, 100, 0), (1, 12, 166_375, 50, 0), (1, 16, 62_400, 50, 0)]
+WIDE_FASTER = [
+    (1, 5, 198_476, 20, 1), (2, 5, 1_376_256, 20, 1), (1, 8, 499_280, 20, 1), (1, 8, 2_000_376, 50, 1),
+    (2, 8, 576, 10, 1), (1, 10, 796_000, 50, 1), (1, 14, 287_496, 50, 1), (1, 17, 59_582, 50, 1),
+    (1, 24, 83_248, 50, 1), (1, 32, 125_000, 32, 1), (2, 4, 1_003_520, 20, 0), (1, 3, 2_666_000, 50, 0),
+    (1, 6, 1_331_000, 20, 0), (1, 8, 1_000_000, 20, 0), (1, 1, 4_000_000, 20, 0), (1, 12, 333_270, 20, 0)]
+
+
+def test_soft_forward_takes_the_faster_kernel(lib) -> None:
+    for b, c, n, k, labels in GENERIC_FASTER:
+        assert not lib.soft_forward_wide(b, c, n, k, 1, labels), (b, c, n, k, labels)
+    for b, c, n, k, labels in WIDE_FASTER:
+        assert lib.soft_forward_wide(b, c, n, k, 1, labels), (b, c, n, k, labels)
+
+
+def test_soft_forward_rule_above_some_size(lib) -> None:
+    """From some size on the wide kernel takes every larger problem of up to 50
+    bins, and above 16 channels every problem."""
+    for c in (1, 2, 3, 4, 5, 8, 9, 12, 16, 17, 40, 64):
+        for k in (1, 10, 20, 50):
+            wide = [lib.soft_forward_wide(1, c, 4 ** i, k, 1, 0) for i in range(1, 15)]
+            assert wide[-1] and (c <= 16 or all(wide)), (c, k, wide)
+            # a problem too small for many blocks may be wide too
+            assert sum(a != b for a, b in zip(wide, wide[1:])) <= 2, (c, k, wide)
 
 
 def _spills(path: Path) -> dict:

@@ -83,6 +83,13 @@ void wide_geometry(long long B, long long C, long long N, int K, int soft, int b
   out[8] = (long long)(g.nt / g.copies) * g.steps * g.var.vec;
 }
 
+// 1: the wide kernel takes the soft forward, 0: the generic one.
+int soft_forward_wide(long long B, long long C, long long N, int K, int bg, int labels) {
+  const ace::Geometry w = ace::make_wide_geometry(B, C, N, K, true, bg != 0, labels != 0, 4, false);
+  const ace::Geometry g = ace::make_geometry(B, C, N, K, true, bg != 0, labels != 0);
+  return ace::wide_soft_forward_pays(w, g, labels != 0) ? 1 : 0;
+}
+
 int exact_shift(long long voxels, int first) {
   return first ? ace::exact_moment_shift0(voxels) : ace::exact_moment_shift(voxels);
 }
