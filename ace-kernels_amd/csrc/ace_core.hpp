@@ -1733,9 +1733,9 @@ static __device__ __align__(16) unsigned char g_dummy_src[64];
 
 // Element v of a row.  SC: a uniform pointer plus an unsigned 32-bit byte offset,
 // the address form that takes the row from scalar registers (no vector
-// arithmetic per row and access).  Every backward and the 16-channel forward
-// use it (soft bf16 32 x 4 x 512^2 backward: 37.4 -> 36.0 us); in the forward at
-// four channels and fewer the addresses are a few instructions in a loop that
+// arithmetic per row and access).  The backward (scalar_rows) and the
+// 16-channel forward use it (soft bf16 32 x 4 x 512^2 backward: 37.4 -> 36.0 us);
+// in the forward at four channels and fewer the addresses are a few instructions in a loop that
 // waits for its loads, and their other form left the scheduler the better
 // order (hard 2 x 4 x 128^3, a pass: 47.3 us against 49.5).
 template <bool SC, typename T>
@@ -1743,6 +1743,15 @@ __device__ __forceinline__ T* row_at(T* row, uint32_t v) {
   if constexpr (!SC) return row + v;
   using Byte = typename std::conditional<std::is_const<T>::value, const char, char>::type;
   return reinterpret_cast<T*>(reinterpret_cast<Byte*>(row) + v * (uint32_t)sizeof(T));
+}
+
+// The backward's choice: not the 16-channel soft gradient of 16-bit logits, one
+// 2-byte element per lane and row, whose loads the scheduler then no longer kept
+// ahead of the arithmetic (1 x 16 x 128^3 bf16: K = 20 41.5 -> 56.8 us, K = 50
+// 54.3 -> 100.9, without background 71.9 -> 167; 40.4, 52.4 and 66.8 this way).
+template <typename T, int C, bool SOFT>
+constexpr bool scalar_rows() {
+  return C <= 4 || !SOFT || sizeof(T) == 4;
 }
 
 template <int C, int VEC>
@@ -2288,6 +2297,7 @@ template <typename T, int C, int VEC, bool SOFT, bool RIGHT, bool SKIP0, bool ST
 __device__ __forceinline__ void bwd_fast_body(const BwdParams& P, const int64_t blk,
                                               unsigned char* smem) {
   float* tabs = reinterpret_cast<float*>(smem);
+  constexpr bool kScalarRows = scalar_rows<T, C, SOFT>();
   const int K = P.K;
   const int n = SOFT ? 2 * K : K;
   constexpr int off = SKIP0 ? 1 : 0;
@@ -2348,9 +2358,9 @@ __device__ __forceinline__ void bwd_fast_body(const BwdParams& P, const int64_t 
 #pragma unroll
     for (int c = 0; c < C; ++c) px[c] = pipe ? xr[c] : reinterpret_cast<const T*>(g_dummy_src);
     const long long* pl = pipe ? lr_ : reinterpret_cast<const long long*>(g_dummy_src);
-    fast_load<T, C, VEC, false, true>(ta, px, pl, pipe ? at(0) : 0u, SOFT);
+    fast_load<T, C, VEC, false, kScalarRows>(ta, px, pl, pipe ? at(0) : 0u, SOFT);
     keep_order<C>();
-    fast_load<T, C, VEC, false, true>(tb, px, pl, pipe ? at(1) : 0u, SOFT);
+    fast_load<T, C, VEC, false, kScalarRows>(tb, px, pl, pipe ? at(1) : 0u, SOFT);
     keep_order<C>();
   }
   treg.store(tabs, P.btab, P.rtab, n, nrepl, kThreads);
@@ -2386,27 +2396,27 @@ __device__ __forceinline__ void bwd_fast_body(const BwdParams& P, const int64_t 
     for (; i + 2 < nsteps; i += 2) {
       fast_backward<C, VEC, SOFT, RIGHT, SKIP0>(ta, tab, sab, scoef, sg, K);
 #pragma unroll
-      for (int c = 0; c < C; ++c) store_dx<T, VEC, STREAM>(row_at<true>(dr[c], at(i)), ta.x[c]);
-      fast_load<T, C, VEC, false, true>(ta, xr, lr_, at(i + 2), SOFT);
+      for (int c = 0; c < C; ++c) store_dx<T, VEC, STREAM>(row_at<kScalarRows>(dr[c], at(i)), ta.x[c]);
+      fast_load<T, C, VEC, false, kScalarRows>(ta, xr, lr_, at(i + 2), SOFT);
       keep_order<C>();
       fast_backward<C, VEC, SOFT, RIGHT, SKIP0>(tb, tab, sab, scoef, sg, K);
 #pragma unroll
-      for (int c = 0; c < C; ++c) store_dx<T, VEC, STREAM>(row_at<true>(dr[c], at(i + 1)), tb.x[c]);
-      fast_load<T, C, VEC, false, true>(tb, xr, lr_, at(i + 3), SOFT);
+      for (int c = 0; c < C; ++c) store_dx<T, VEC, STREAM>(row_at<kScalarRows>(dr[c], at(i + 1)), tb.x[c]);
+      fast_load<T, C, VEC, false, kScalarRows>(tb, xr, lr_, at(i + 3), SOFT);
       keep_order<C>();
     }
     fast_backward<C, VEC, SOFT, RIGHT, SKIP0>(ta, tab, sab, scoef, sg, K);
 #pragma unroll
-    for (int c = 0; c < C; ++c) store_dx<T, VEC, STREAM>(row_at<true>(dr[c], at(i)), ta.x[c]);
+    for (int c = 0; c < C; ++c) store_dx<T, VEC, STREAM>(row_at<kScalarRows>(dr[c], at(i)), ta.x[c]);
     if (i + 1 < nsteps) {
       fast_backward<C, VEC, SOFT, RIGHT, SKIP0>(tb, tab, sab, scoef, sg, K);
 #pragma unroll
-      for (int c = 0; c < C; ++c) store_dx<T, VEC, STREAM>(row_at<true>(dr[c], at(i + 1)), tb.x[c]);
+      for (int c = 0; c < C; ++c) store_dx<T, VEC, STREAM>(row_at<kScalarRows>(dr[c], at(i + 1)), tb.x[c]);
     }
   }
   for (int v = nsteps * stride + tid * VEC; v < nfull; v += stride) {
     FastTile<C, VEC> t;
-    fast_load<T, C, VEC, false, true>(t, xr, lr_, (uint32_t)v, SOFT);
+    fast_load<T, C, VEC, false, kScalarRows>(t, xr, lr_, (uint32_t)v, SOFT);
     fast_backward<C, VEC, SOFT, RIGHT, SKIP0>(t, tab, sab, scoef, sg, K);
 #pragma unroll
     for (int c = 0; c < C; ++c) store_dx<T, VEC, STREAM>(dr[c] + v, t.x[c]);
