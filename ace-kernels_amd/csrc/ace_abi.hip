@@ -302,7 +302,6 @@ FwdParams fwd_params(const void* x, int x_dtype, const void* target, bool labels
   p.empty_w = empty_weight;
   p.packed = g.packed ? 1 : 0;
   p.right = right;
-  p.tl = g_timeline.load(std::memory_order_relaxed);
   p.max_polls = g_max_polls.load(std::memory_order_relaxed);
   p.publish_delay = g_publish_delay.load(std::memory_order_relaxed);
   p.pscale = 1.0 / 1073741824.0;  // the generic kernels' sums: 30-bit fixed point
@@ -567,10 +566,12 @@ int ace_forward(const void* x, int x_dtype, const void* target, int target_kind,
   const bool moments = fp.moments;
   if (workspace_bytes < g.ws_bytes) return ACE_EWORKSPACE;
 
-  const FwdParams p = fwd_params(x, x_dtype, target, labels, voxels, batch, channels, num_bins, act,
-                                  ignore_empty_classes, reduction, right != 0, empty_weight, moments,
-                                  class_weight, bin_table, centre_table, workspace, g, coef, diff, jac, per_class,
-                                  loss, stats);
+  FwdParams p = fwd_params(x, x_dtype, target, labels, voxels, batch, channels, num_bins, act,
+                           ignore_empty_classes, reduction, right != 0, empty_weight, moments,
+                           class_weight, bin_table, centre_table, workspace, g, coef, diff, jac, per_class,
+                           loss, stats);
+  // the buffer holds the blocks of the fast launches it was set for, no others
+  if (g.fast) p.tl = g_timeline.load(std::memory_order_relaxed);
   return to_code(dispatch_fwd(x_dtype, soft, right != 0, g, p, static_cast<hipStream_t>(stream)));
 }
 

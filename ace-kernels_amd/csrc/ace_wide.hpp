@@ -241,7 +241,6 @@ constexpr int wide_min_waves(int C) { return C <= 16 ? 4 : (C <= 32 ? 3 : 2); }
 template <typename T, int C, int CMIN, int VEC, bool SOFT, bool LABELS>
 __global__ void __launch_bounds__(kThreads, (wide_min_waves(C))) fwd_kernel_wide(const FwdParams P) {
   extern __shared__ __align__(16) unsigned char smem[];
-  fast_stamp(P, kTlStart);
   float* tabs = reinterpret_cast<float*>(smem);
   const int K = P.K;
   const int n = SOFT ? 2 * K : K;
@@ -323,7 +322,6 @@ __global__ void __launch_bounds__(kThreads, (wide_min_waves(C))) fwd_kernel_wide
     load(tb, v + 3 * stride);
   }
   __syncthreads();
-  fast_stamp(P, kTlLoop);
   constexpr int kMom = !SOFT ? kMomNone : (LABELS ? kMomExact : kMomExactTargets);
   fwd_finish<SOFT, kMom, kMaxWideCopies>(P, H, hist, repl, CK, CL, b, tile, LABELS);
 }

@@ -277,7 +277,8 @@ int ace_set_launch_events(void* start, void* stop);
  * (s_memrealtime) at its phases: 0 start, 1 main loop done, 2 block sums and
  * their final-sum atomics done, 3 ticket drawn, and in the blocks that run
  * an epilogue 4 epilogue done, 5 loss written, 6 soft moments' terms done,
- * 7 bins done.  The buffer must hold the launch's blocks; process-wide.
+ * 7 bins done.  The buffer must hold the launch's blocks; process-wide.  No
+ * other launch (other kernels, ace_forward_levels) writes to it.
  * Returns ACE_OK.
  */
 size_t ace_read_bytes_scratch(void);
