@@ -82,6 +82,9 @@ hipError_t dispatch_bwd(int dtype, bool soft, bool right, const Geometry& g, con
 namespace {
 
 constexpr size_t kMaxLds = 160 * 1024;  // gfx950 LDS per workgroup
+// Of a forward: beside its dynamic LDS it has a static word (fwd_finish), which
+// takes 16 bytes.
+constexpr size_t kMaxFwdLds = kMaxLds - 16;
 
 size_t elem_size(int dtype) { return dtype == ACE_F32 ? 4 : 2; }
 
@@ -136,7 +139,7 @@ bool use_moments(bool soft, bool labels, int act, int64_t batch, int64_t channel
     return false;
   const Geometry g = make_geometry(batch, channels, voxels, num_bins, true, include_background != 0,
                                    true, 0, 0, true, true, kThreads);
-  return g.lds_fwd <= kMaxLds && g.lds_bwd <= kMaxLds;
+  return g.lds_fwd <= kMaxFwdLds && g.lds_bwd <= kMaxLds;
 }
 
 // The forward runs a fast kernel (fast_bins, 1024-thread blocks where the
@@ -195,7 +198,7 @@ Geometry wide_geometry(bool soft, bool labels, int act, int64_t batch, int64_t c
   if (act == kActNone || channels > kMaxChannels || (soft && num_bins > kExactMaxBins)) return g;
   g = make_wide_geometry(batch, channels, voxels, num_bins, soft, include_background != 0, labels,
                          elem_size(x_dtype), backward);
-  g.wide = voxels >= g.var.vec && g.lds_fwd <= kMaxLds && g.lds_bwd <= kMaxLds && g.nblk <= 0x7fffffffLL;
+  g.wide = voxels >= g.var.vec && g.lds_fwd <= kMaxFwdLds && g.lds_bwd <= kMaxLds && g.nblk <= 0x7fffffffLL;
   return g;
 }
 
@@ -243,7 +246,7 @@ ForwardPlan plan_forward(int64_t batch, int64_t channels, int64_t voxels, int nu
   fp.moments = use_moments(soft, labels, fp.act, batch, channels, voxels, num_bins, include_background);
   fp.g = forward_geometry(batch, channels, voxels, num_bins, soft, include_background, labels, fp.act,
                           fp.moments);
-  fp.rc = (fp.g.lds_fwd > kMaxLds || fp.g.nblk > 0x7fffffffLL) ? ACE_EUNSUPPORTED : ACE_OK;
+  fp.rc = (fp.g.lds_fwd > kMaxFwdLds || fp.g.nblk > 0x7fffffffLL) ? ACE_EUNSUPPORTED : ACE_OK;
   if (!fast_forward(soft, labels, fp.act, channels, fp.moments)) {
     const Geometry w =
         wide_geometry(soft, labels, fp.act, batch, channels, voxels, num_bins, include_background, x_dtype);
@@ -664,7 +667,7 @@ int ace_forward_levels(int levels, const AceFwdLevel* lv, int x_dtype, int64_t b
     if (soft && !moments) return ACE_EUNSUPPORTED;
     const Geometry g = forward_geometry(batch, channels, v.voxels, num_bins, soft,
                                         include_background, true, kActSoftmax, moments, max_nt);
-    if (g.lds_fwd > kMaxLds) return ACE_EUNSUPPORTED;
+    if (g.lds_fwd > kMaxFwdLds) return ACE_EUNSUPPORTED;
     // one launch, one block size: every level's geometry must use it
     if (g.nt != L.nt) return ACE_EUNSUPPORTED;
     if (nblk + g.nblk > 0x7fffffffLL) return ACE_EUNSUPPORTED;

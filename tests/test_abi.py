@@ -182,6 +182,30 @@ def test_f64_forward_refuses_lds_beside_its_static_arrays() -> None:
         assert lib.ace_forward_f64(*args) == 2, k  # ACE_EUNSUPPORTED
 
 
+def test_forward_refuses_lds_beside_its_static_word() -> None:
+    """A forward whose dynamic LDS fits the 160 KiB workgroup alone but not
+    beside the kernel's static word (16 bytes) is refused before any HIP call.
+    Hard binning with labels, C = 5 without background: bucket table and
+    epilogue take exactly 160 KiB at 2925 bins (sigmoid and softmax alike).  Only
+    refused configurations are called here (fake pointers)."""
+    lib = _lib.lib()
+    fake, limit = 256, 160 * 1024
+
+    def dyn_lds(k, classes):
+        ck = classes * k
+        epilogue = ((13 * ck + 15) // 16 * 16 + 4 * classes + 15) // 16 * 16
+        return ((k + 2 + 3) // 4 * 4) * 4 + max(epilogue, (8 * ck + 15) // 16 * 16)
+
+    assert dyn_lds(2925, 4) == limit
+    for act in (_lib.ACT_SOFTMAX, _lib.ACT_SIGMOID):
+        args = [fake, _lib.F32, fake, _lib.TARGET_LABELS_I64, 2, 5, 4096, 2925, _lib.HARD, act,
+                0, 1, _lib.RED_MEAN, 0, 0.01, None, fake, None, fake, 1 << 40, fake, fake, fake, fake,
+                fake, None, None]
+        assert lib.ace_forward(*args) == _lib.EUNSUPPORTED
+        noalloc = args[:18] + args[20:]
+        assert lib.ace_forward_noalloc(*noalloc) == _lib.EUNSUPPORTED
+
+
 def test_f64_entry_points_validate_before_launch() -> None:
     """ace_forward_f64 / ace_backward_f64 reject bad arguments before any HIP
     call; ace_workspace_bytes sizes their workspace for x_dtype ACE_F64."""
