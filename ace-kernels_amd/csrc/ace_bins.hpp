@@ -175,7 +175,7 @@ ACE_HD MomentScale moment_scale(int num_bins) {
 
 // Exact moments (the wide soft kernels, any p): the probabilities of half-bin
 // h are held as u = p 2^m - h w, exact in float32 and, for h >= 1, an integer
-// below 2^25:
+// below 1.2 2^24:
 //   m = 23 + ceil(log2 2K): p > 1/2K (1 - 2^-14) there, whose spacing is at
 //   least 2^-m;
 //   ws = 2^m / 2K is in [2^23, 2^24), and w <= ws (1 - 2^-14) has at most
@@ -200,13 +200,14 @@ ACE_HD MomentScale exact_moment_scale(int num_bins) {
   s.w = ((int)(ws * (1.0 - 1.0 / 16384.0)) >> drop) << drop;
   return s;
 }
-// Right shifts of its per-copy sums before the final sums of N voxels: u^2 <
-// 2^50.6 (a copy's 4095 voxels below 2^62.6), N 2^50.6 / 2^shift < 2^62.6; and
-// of half-bin 0's sums, 2^16 u < 2^40 a voxel.
+// Right shifts of its per-copy sums before the final sums of N voxels, as few
+// bits as keep these inside int64: u < 1.2 2^24, so u^2 < 2^48.6 (a copy's 4095
+// voxels below 2^60.6) and N 2^48.6 / 2^shift < 2^62.6; and of half-bin 0's sums,
+// 2^16 u < 2^40 (1 + 2^-13) a voxel.
 ACE_HD int exact_moment_shift(long long voxels) {
   int bits = 0;
   while (bits < 62 && (1ll << bits) <= voxels) ++bits;
-  return bits > 12 ? bits - 12 : 0;
+  return bits > 14 ? bits - 14 : 0;
 }
 ACE_HD int exact_moment_shift0(long long voxels) {
   int bits = 0;

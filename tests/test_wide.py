@@ -63,6 +63,9 @@ def test_shifts(lib) -> None:
         n = (1 << bits) - 1
         assert n * 1.2 ** 2 * 2 ** 48 / 2 ** lib.exact_shift(n, 0) < 2 ** 63
         assert n * 2 ** 40 / 2 ** lib.exact_shift(n, 1) < 2 ** 63
+        # and no bit of the squares is dropped that could stay
+        shift = lib.exact_shift(n, 0)
+        assert shift == 0 or (n + 1) * 1.2 ** 2 * 2 ** 48 / 2 ** (shift - 1) > 2 ** 63
 
 
 @pytest.mark.parametrize("soft", [0, 1])

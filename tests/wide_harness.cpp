@@ -28,7 +28,7 @@ extern "C" {
 // every p within `width` ulp of the 2K upper half boundaries `table`: with h
 // the half-bin, u = fma(p, 2^m, -(h w)) in float32 must equal the exact
 // p 2^m - h w (double holds it), be non-negative and below `umax`, and for
-// h >= 1 be an integer.  w_div > 1 plants a base that keeps too many bits.
+// h >= 1 be an integer.  plant != 0 plants a base that keeps too many bits.
 long long check_exact_moments(const float* table, int num_bins, int width, int step, double umax,
                               int plant) {
   ace::MomentScale s = ace::exact_moment_scale(num_bins);
