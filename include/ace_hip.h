@@ -75,6 +75,10 @@ const char* ace_error_string(int code);
  * reuse a workspace without clearing.  A call that needs more reset bytes than
  * earlier calls on the same buffer have left zero needs the extra bytes
  * cleared first.  Calls that share a workspace must be ordered (same stream).
+ * ace_forward also takes a smaller workspace that holds the generic kernels'
+ * sums (three words per bin instead of up to eleven), and then runs those
+ * kernels, which are slower at most sizes; below that it returns
+ * ACE_EWORKSPACE.
  */
 size_t ace_workspace_bytes(int64_t batch, int64_t channels, int64_t voxels,
                            int num_bins, int binning, int x_dtype,
@@ -122,7 +126,8 @@ int ace_forward(const void* x, int x_dtype, const void* target,
  * values; a caller holding only a float32 d passes zeros as its remainder);
  * `diff` may be NULL for hard binning.
  * `target` may be NULL for hard binning (the hard gradient does not use it).
- * dx has the element type of x.
+ * dx has the element type of x and must not overlap it: some kernels read and
+ * store the last voxels of a row in two lanes.
  */
 int ace_backward(const void* x, int x_dtype, const void* target,
                  int target_kind, int64_t batch, int64_t channels,
@@ -226,9 +231,9 @@ int ace_backward_levels(int levels, const AceBwdLevel* lv, int x_dtype,
  * device, held until the process ends) instead of an argument; it calls no
  * allocating routine.  The array used is the current device's (x and the
  * outputs must live there).  Before the forward it clears the bytes the
- * problem needs with a fill kernel on `stream`.  Problems whose
- * ace_workspace_bytes() exceed ACE_NOALLOC_SCRATCH_BYTES return ACE_ESCRATCH
- * before any launch.  Every call on a device shares that device's array:
+ * problem needs with a fill kernel on `stream`.  Problems that need more than
+ * ACE_NOALLOC_SCRATCH_BYTES even for the generic kernels' sums (see
+ * ace_workspace_bytes) return ACE_ESCRATCH before any launch.  Every call on a device shares that device's array:
  * calls that overlap on one device (different streams, or threads without an
  * order between them) race and must be serialised by the caller.
  */
