@@ -81,10 +81,11 @@ def test_steps(binning, voxels) -> None:
 
 @pytest.mark.parametrize("binning", ["hard", "soft"])
 @pytest.mark.parametrize("channels", [5, 9])
-def test_extreme_logits(binning, channels) -> None:
-    """Voxels with infinite, NaN or very large logits leave every other voxel's
-    gradient as it is without them, up to the sums they count in; saturated
-    voxels match the reference."""
+def test_extreme_logits(channels, binning) -> None:
+    """Saturated voxels match the reference; voxels with infinite or NaN logits
+    leave every other voxel's gradient as it is with ordinary logits of the same
+    probabilities in their place (a NaN or minus infinity beside finite logits:
+    probability 0; plus infinity: all equal), and the loss too."""
     gen = torch.Generator().manual_seed(3)
     x = torch.randn(1, channels, 2000, generator=gen)
     x[0, :, ::7] *= 400.0
@@ -92,9 +93,54 @@ def test_extreme_logits(binning, channels) -> None:
     cfg = ACEConfig(binning=binning, num_bins=10, to_onehot_y=True)
     say(f"wide extreme {binning} C={channels}")
     _check(x, y, cfg)
+    # 12 bins: 1 / 5 and 1 / 9 lie far from every edge and centre
+    cfg = ACEConfig(binning=binning, num_bins=12, to_onehot_y=True)
+    x[0, :, 5:8] = torch.randn(channels, 3, generator=gen)
+    low = x.clone()
     x[0, 0, 5], x[0, 1, 6], x[0, 2, 7] = float("inf"), float("-inf"), float("nan")
+    low[0, :, 5], low[0, 1, 6], low[0, 2, 7] = 0.25, -1000.0, -1000.0
     loss, grad = run("hip_mi355x", x.cuda(), y.cuda(), cfg)
-    assert bool(torch.isfinite(loss)) and bool(torch.isfinite(grad[0, :, 8:]).all())
+    loss_low, grad_low = run("hip_mi355x", low.cuda(), y.cuda(), cfg)
+    torch.testing.assert_close(loss, loss_low, rtol=1e-6, atol=0)
+    # hard: coefficients are counts and signs; soft: d moves by the last bit of
+    # the equal probabilities
+    others = torch.ones(2000, dtype=torch.bool)
+    others[5:8] = False
+    got, want = grad[0, :, others], grad_low[0, :, others]
+    if binning == "hard":
+        assert torch.equal(got, want)
+    else:
+        torch.testing.assert_close(got, want, rtol=1e-5, atol=1e-9)
+
+
+@pytest.mark.parametrize("binning", ["hard", "soft"])
+@pytest.mark.parametrize("dtype,channels,voxels", [
+    (torch.float32, 5, 1_100_003), (torch.bfloat16, 7, 1_700_001), (torch.float16, 13, 800_005),
+    (torch.bfloat16, 21, 600_001), (torch.float32, 15, 2_100_001)])
+def test_many_steps(dtype, channels, voxels, binning) -> None:
+    """Blocks of several steps (two tiles in rotation, a row's end after full
+    steps), 16-bit logits, and (the last one, 273 MB of logits, labels and
+    gradient) streaming stores: the gradient equals to the bit that of pieces whose blocks
+    take one step, from the same coefficients, and the hard forward's sums are
+    the pieces' sums."""
+    gen = torch.Generator(device="cuda").manual_seed(voxels)
+    x = (torch.randn(1, channels, voxels, generator=gen, device="cuda") * 2.0).to(dtype)
+    y = torch.randint(0, channels, (1, 1, voxels), generator=gen, device="cuda")
+    cfg = ACEConfig(binning=binning, num_bins=20, to_onehot_y=True)
+    say(f"wide many steps {binning} {dtype} C={channels} N={voxels}")
+    go = torch.ones((), device="cuda")
+    pl = hip.make_plan(x, y, cfg)
+    _, coef, d, jac, _, st = hip.hip_forward(pl, cfg, stats=True)
+    grad = hip.hip_backward(pl, coef, d, jac, go)
+    total, at = torch.zeros_like(st), 0
+    while at < voxels:
+        n = min(99_991, voxels - at)
+        piece = hip.make_plan(x[:, :, at:at + n].contiguous(), y[:, :, at:at + n].contiguous(), cfg)
+        total += hip.hip_forward(piece, cfg, stats=True)[5]
+        assert torch.equal(hip.hip_backward(piece, coef, d, jac, go), grad[:, :, at:at + n]), at
+        at += n
+    if binning == "hard":
+        assert torch.equal(total, st)
 
 
 def _stats(x, y, cfg, ws_bytes):

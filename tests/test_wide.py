@@ -74,15 +74,19 @@ def test_shifts(lib) -> None:
 @pytest.mark.parametrize("backward", [0, 1])
 def test_geometry(lib, soft, labels, elem, backward) -> None:
     """Every channel count has a variant that holds it; no copy counts more
-    voxels than its field; the tiles cover the row; the hard layout needs no
-    more workspace than the generic kernels' (same final sums)."""
+    voxels than its field; the tiles cover the row; the LDS of both kernels at
+    20 bins fits; and the workspace holds the final sums of every replica."""
     out = (ctypes.c_longlong * 9)()
     for c in range(1, 65):
         for n in (0, 1, 255, 256, 257, 20001, 128 ** 3):
             for k in (1, 20, 50, 512):
                 for b, bg in ((1, 1), (3, 0)):
                     lib.wide_geometry(b, c, n, k, soft, bg, labels, elem, backward, out)
-                    cmax, vec, copies, steps, _, _, tiles, _, count = out
+                    cmax, vec, copies, steps, lds_fwd, lds_bwd, tiles, ws_bytes, count = out
+                    if k <= 20:
+                        assert lds_fwd <= MAX_LDS - 16 and lds_bwd <= MAX_LDS
+                    words = (10 if labels else 11) if soft else (2 if labels else 3)
+                    assert ws_bytes >= b * words * (c - (1 - bg if c > 1 else 0)) * k * 8
                     assert c <= cmax <= max(c + 1, 1.46 * c) and vec in (1, 2, 4)
                     assert copies in (1, 2, 4, 8) and steps >= 1
                     assert count <= (4095 if soft else 2047), (c, n, k, count)
