@@ -365,7 +365,10 @@ constexpr int wide_vec(int cmax, size_t elem, bool soft, bool labels, bool backw
   if (labels) return elem == 2 || cmax <= 16 ? 2 : 1;
   return cmax <= 8 ? 2 : 1;
 }
-constexpr size_t kMaxWideHistLds = 39 * 1024;  // four blocks per CU with their tables
+// LDS of the histogram copies: four blocks per CU with their tables, unless a
+// soft forward's epilogue (109 bytes per bin, in the same region) or a single
+// copy takes more.
+constexpr size_t kMaxWideHistLds = 39 * 1024;
 constexpr int kMaxWideCopies = 8;
 
 inline Geometry make_wide_geometry(int64_t B, int64_t C, int64_t N, int K, bool soft,

@@ -1,7 +1,9 @@
 // Wide kernels: the loss's forward and backward for any channel count up to
 // 64, softmax or sigmoid, class labels or per-channel targets, hard binning
 // and soft binning in the moments layout.  They serve every such call that
-// the fast kernels (softmax, class labels, C in {2, 3, 4, 16}) do not.
+// the fast kernels (softmax, class labels, C in {2, 3, 4, 16}) do not, but for
+// the soft forwards of few voxels with many bins, where the generic kernels are
+// the faster ones (wide_soft_forward_pays).
 //
 // A lane takes one to four voxels a step (wide_vec), one after the other, all
 // channels of a voxel in registers.  The channel count is a compile-time CMAX with
